@@ -47,16 +47,12 @@
 
 #include "dkz_device.hpp"
 #include "dkz_internal.hpp"
+#include "gemm_split.hpp"
 
 namespace dkz {
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int kBK = 16;
 constexpr int kPitch = kBK + 4;  // LDS row pitch in words
-constexpr int kGroupM = 8;
-constexpr int kXcds = 8;
 
 // Slabs in flight in the 64x64 kernel (build-time tunable).
 #ifndef DKZ_GEMM_SMALL_PREFETCH
@@ -706,16 +702,10 @@ __global__ __launch_bounds__(kBlock, 4) void gemm_mfma_kernel(GemmArgs g) {
 // The split-K epilogue: C(i, j) = beta-applied C + alpha * (sum of the splits'
 // partials in split order). V4: n % 4 == 0 and C's rows are float4-aligned,
 // so a lane takes four consecutive columns of one row.
-__device__ __forceinline__ float gemm_out(const float *cp, float s, const GemmArgs &g) {
-    float cv = 0.0f;
-    if (g.beta != 0.0f) cv = (g.beta == 1.0f) ? *cp : *cp * g.beta;
-    return cv + g.alpha * s;
-}
-
 constexpr int kReduceBatch = 8;
 
-template <bool V4>
-__global__ __launch_bounds__(kBlock) void gemm_splitk_reduce_kernel(GemmArgs g) {
+template <bool V4, class Args>
+__global__ __launch_bounds__(kBlock) void gemm_splitk_reduce_kernel(Args g) {
     const uint32_t mn = g.m * g.n;
     if constexpr (V4) {
         const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
@@ -739,8 +729,8 @@ __global__ __launch_bounds__(kBlock) void gemm_splitk_reduce_kernel(GemmArgs g) 
             }
         }
         float *cp = g.c + i * g.ldc + j;
-        const float4 o = make_float4(gemm_out(cp, s.x, g), gemm_out(cp + 1, s.y, g), gemm_out(cp + 2, s.z, g),
-                                     gemm_out(cp + 3, s.w, g));
+        const float4 o = make_float4(gemm_out(cp, s.x, g.alpha, g.beta), gemm_out(cp + 1, s.y, g.alpha, g.beta),
+                                     gemm_out(cp + 2, s.z, g.alpha, g.beta), gemm_out(cp + 3, s.w, g.alpha, g.beta));
         *reinterpret_cast<float4 *>(cp) = o;
     } else {
         const uint32_t e = blockIdx.x * kBlock + threadIdx.x;
@@ -755,19 +745,28 @@ __global__ __launch_bounds__(kBlock) void gemm_splitk_reduce_kernel(GemmArgs g) 
             for (int u = 0; u < kReduceBatch; ++u) s += p[u];
         }
         float *cp = g.c + i * g.ldc + j;
-        *cp = gemm_out(cp, s, g);
+        *cp = gemm_out(cp, s, g.alpha, g.beta);
     }
 }
 
-template <int BM, int BN, int D>
-int launch_gemm(bool ta, bool tb, GemmArgs g) {
+// Adds the splits' partial tiles into C.
+template <class Args>
+int launch_reduce(const char *name, const Args &g) {
+    const uint64_t mn = (uint64_t)g.m * g.n;
+    if (g.n % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.c))
+        return launch(name, gemm_splitk_reduce_kernel<true, Args>, dim3(div_up(mn / 4, kBlock)), dim3(kBlock), g);
+    return launch(name, gemm_splitk_reduce_kernel<false, Args>, dim3(div_up(mn, kBlock)), dim3(kBlock), g);
+}
+
+template <int BM, int BN>
+int launch_gemm(bool ta, bool tb, const SplitArgs &g) {
     const uint64_t total = (uint64_t)g.tiles_m * g.tiles_n * g.splits;
     DKZ_REQUIRE(total <= 0x7fffffffull);
     const dim3 grid((uint32_t)total), block(kBlock);
-    if (!ta && !tb) return launch("gemm_nn", gemm_mfma_kernel<BM, BN, false, false, D>, grid, block, g);
-    if (ta && !tb) return launch("gemm_tn", gemm_mfma_kernel<BM, BN, true, false, D>, grid, block, g);
-    if (!ta && tb) return launch("gemm_nt", gemm_mfma_kernel<BM, BN, false, true, D>, grid, block, g);
-    return launch("gemm_tt", gemm_mfma_kernel<BM, BN, true, true, D>, grid, block, g);
+    if (!ta && !tb) return launch("gemm_nn", gemm_split_kernel<BM, BN, kRowMajor, kColMajor>, grid, block, g);
+    if (ta && !tb) return launch("gemm_tn", gemm_split_kernel<BM, BN, kColMajor, kColMajor>, grid, block, g);
+    if (!ta && tb) return launch("gemm_nt", gemm_split_kernel<BM, BN, kRowMajor, kRowMajor>, grid, block, g);
+    return launch("gemm_tt", gemm_split_kernel<BM, BN, kColMajor, kRowMajor>, grid, block, g);
 }
 
 // A batched NN product over z = 0 .. zcount-1 (one grid row each); IM != kImNone:
@@ -919,12 +918,7 @@ int launch_wgrad(const GemmArgs &g) {
     const dim3 grid(g.tiles_m * g.tiles_n * g.splits);
     constexpr int D = BM == 128 ? 1 : DKZ_GEMM_SMALL_PREFETCH;
     DKZ_TRY(launch("convolution_weight_gradient", gemm_mfma_kernel<BM, BM, false, true, D, IM>, grid, dim3(kBlock), g));
-    if (g.splits == 1) return 0;
-    if (g.n % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.c))
-        return launch("convolution_weight_gradient", gemm_splitk_reduce_kernel<true>,
-                      dim3(div_up((uint64_t)g.m * g.n / 4, kBlock)), dim3(kBlock), g);
-    return launch("convolution_weight_gradient", gemm_splitk_reduce_kernel<false>,
-                  dim3(div_up((uint64_t)g.m * g.n, kBlock)), dim3(kBlock), g);
+    return g.splits == 1 ? 0 : launch_reduce("convolution_weight_gradient", g);
 }
 
 template <int IM>
@@ -959,7 +953,7 @@ int dkz_gemm(int ta, int tb, int m, int n, int k, float alpha, const float *a, i
         DKZ_REQUIRE(extent(ta ? k : m, ta ? m : k, lda) + 3 <= kMaxElems);
         DKZ_REQUIRE(extent(tb ? n : k, tb ? k : n, ldb) + 3 <= kMaxElems);
     }
-    GemmArgs g{};
+    SplitArgs g{};
     g.a = a;
     g.b = b;
     g.c = c;
@@ -971,20 +965,33 @@ int dkz_gemm(int ta, int tb, int m, int n, int k, float alpha, const float *a, i
     g.ldc = (uint32_t)ldc;
     g.alpha = alpha;
     g.beta = beta;
-    g.vec_a = aligned16(a) && lda % 4 == 0;
-    g.vec_b = aligned16(b) && ldb % 4 == 0;
     g.splits = 1;
     g.k_chunk = (uint32_t)k;
     g.zgroups = 1;
 
-    // 128x128 tiles when they give every CU two workgroups; 64x64 below, and
-    // if even those leave CUs idle and K is long, split K (ranges of >= 128)
-    // until about DKZ_GEMM_SPLIT_TARGET workgroups per CU, within the scratch.
+    // 128x128 tiles when they give every CU two workgroups, or every CU one
+    // and K in two ranges the second (2048^3: 120 us in one range, 109 in two,
+    // 126 with 64x64 tiles); 64x64 below, and if even those leave CUs idle and K
+    // is long, K in ranges of >= 128 until about DKZ_GEMM_SPLIT_TARGET
+    // workgroups per CU, within the scratch ([256,4096] x [4096,1000]: 26 us
+    // with 64x64 tiles in eight ranges, 29 with 128x64, 30 with 128x128).
+    Scratch sc{};
     const uint64_t big = (uint64_t)div_up(m, 128) * div_up(n, 128);
-    if (big >= 2 * kCus) {
+    if (big >= kCus) {
         g.tiles_m = div_up(m, 128);
         g.tiles_n = div_up(n, 128);
-        return launch_gemm<128, 128, 1>(ta != 0, tb != 0, g);
+        if (big < 2 * kCus && k >= 1024) {
+            DKZ_TRY(device_scratch(&sc));
+            if (2 * (uint64_t)m * n <= sc.gemm_floats) {
+                g.k_chunk = div_up(div_up(k, 2), kBK) * kBK;
+                g.splits = 2;
+                g.partial = sc.gemm;
+            }
+        }
+        if (big >= 2 * kCus || g.splits == 2) {
+            DKZ_TRY((launch_gemm<128, 128>(ta != 0, tb != 0, g)));
+            return g.splits > 1 ? launch_reduce("gemm_splitk_reduce", g) : 0;
+        }
     }
     g.tiles_m = div_up(m, 64);
     g.tiles_n = div_up(n, 64);
@@ -994,7 +1001,6 @@ int dkz_gemm(int ta, int tb, int m, int n, int k, float alpha, const float *a, i
         splits = div_up((uint64_t)DKZ_GEMM_SPLIT_TARGET * kCus, tiles);
         const uint64_t by_k = (uint64_t)k / 128;
         if (splits > by_k) splits = by_k;
-        Scratch sc;
         DKZ_TRY(device_scratch(&sc));
         const uint64_t cap = sc.gemm_floats / ((uint64_t)m * n);
         if (splits > cap) splits = cap;
@@ -1003,19 +1009,10 @@ int dkz_gemm(int ta, int tb, int m, int n, int k, float alpha, const float *a, i
         const uint32_t chunk = (uint32_t)((div_up(k, splits) + kBK - 1) / kBK * kBK);
         g.k_chunk = chunk;
         g.splits = div_up(k, chunk);
-    }
-    if (g.splits > 1) {
-        Scratch sc;
-        DKZ_TRY(device_scratch(&sc));
         g.partial = sc.gemm;
-        DKZ_TRY((launch_gemm<64, 64, DKZ_GEMM_SMALL_PREFETCH>(ta != 0, tb != 0, g)));
-        if (n % 4 == 0 && ldc % 4 == 0 && aligned16(c))
-            return launch("gemm_splitk_reduce", gemm_splitk_reduce_kernel<true>,
-                          dim3(div_up((uint64_t)m * n / 4, kBlock)), dim3(kBlock), g);
-        return launch("gemm_splitk_reduce", gemm_splitk_reduce_kernel<false>, dim3(div_up((uint64_t)m * n, kBlock)),
-                      dim3(kBlock), g);
     }
-    return launch_gemm<64, 64, DKZ_GEMM_SMALL_PREFETCH>(ta != 0, tb != 0, g);
+    DKZ_TRY((launch_gemm<64, 64>(ta != 0, tb != 0, g)));
+    return g.splits > 1 ? launch_reduce("gemm_splitk_reduce", g) : 0;
 }
 
 // convolutional.zig:240-260 in one launch: for image i and group j,
