@@ -17,7 +17,7 @@
 // v_mfma_f32_32x32x2_f32 from the same loads (redo): when an accumulator is
 // not finite (an infinity, a NaN, a value that rounds to a bf16 infinity: its
 // l is a NaN) or when all of a thread's share of some row is tiny (its largest
-// magnitude within (0, 2^-85)). Infinities, NaNs and tiny operands so give
+// magnitude within (0, 2^-100)). Infinities, NaNs and tiny operands so give
 // what fp32 products give.
 //
 // A workgroup of four waves owns a BM x BN tile of C, each wave a quarter of
@@ -49,7 +49,7 @@ constexpr int kGroupM = 8;
 constexpr int kXcds = 8;
 constexpr int kPlanes = 3;
 constexpr int kF32Pitch = kBK + 4;  // LDS row pitch of the fp32 pass, in words
-constexpr float kTiny = 0x1p-85f;
+constexpr float kTiny = 0x1p-100f;
 
 // LDS words of one half (8 k) of a plane of R rows, and of an operand's slab.
 template <int R>
@@ -60,8 +60,33 @@ constexpr int slab_words() { return kPlanes * 2 * half_words<R>(); }
 // Operand kinds. kRowMajor: rows along the tile dimension, k contiguous (A
 // row-major, B transposed). kColMajor: k along the rows, the tile dimension
 // contiguous (A transposed, B row-major), also the (image, position) columns of
-// a 1x1 convolution.
-enum Operand { kRowMajor, kColMajor };
+// a 1x1 convolution. kGather: the same columns of a convolution's im2col, each
+// element read from the image (kGatherWide: images or windows too large for
+// kGather's 32-bit byte offsets and masks). kSeg, kTap: the operands of a weight
+// gradient, whose k runs over (image, position) -- row f of delta (or of a 1x1
+// convolution's input), and a tap's elements (kSegOdd: the positions per image
+// are no multiple of four; kTapWide and kSegWide: 64-bit addresses).
+enum Operand { kRowMajor, kColMajor, kGather, kGatherWide, kSeg, kSegOdd, kTap, kSegWide, kTapWide };
+
+// The image behind a gathered operand: B[k][p] = im2col(image)[k][p] for
+// k = (c, kh, kw) over a group's channels and p = (h, w) over the output
+// positions (im2col.zig:13-49).
+struct ConvGeom {
+    uint32_t H, W, stride, rows, cols;  // rows x cols: the window
+    int32_t pad, pad_x;                 // rows and columns (negative: the window starts inside the image)
+    FastDiv div_kk, div_k, div_wo;      // rows*cols, cols, output width
+};
+
+// One phase of a strided data gradient: its flipped taps (A, `k` = filters x
+// taps per group), their window over delta, and the pixels it writes:
+// (s*yq + py, s*xq + px) for its column (yq, xq).
+struct PhaseDesc {
+    const float *a;
+    uint32_t k, rows, cols, py, px;
+    int32_t pad, pad_x;
+    FastDiv div_kk, div_k;
+};
+constexpr int kMaxPhases = 4;
 
 struct SplitArgs {
     const float *a;
@@ -77,9 +102,33 @@ struct SplitArgs {
     uint64_t a_z, b_z, c_z;
     // Columns over (image, position): npos positions per image (0: one matrix),
     // element strides from one image to the next of B and C.
-    uint32_t npos, b_img, c_img;
+    uint32_t npos;
+    uint64_t b_img, c_img;
     FastDiv div_npos;
+    ConvGeom cv;  // gathered operands and taps only
+    // Weight gradient: positions per image, and those rounded up to a multiple
+    // of four (k = image * kpos4 + position, so that four consecutive k lie in
+    // one image; the positions past kpos read as 0). a_img: delta's element
+    // stride from one image to the next; the input's is b_img.
+    uint32_t kpos;
+    uint64_t a_img;
+    FastDiv div_kpos4;
+    // phases != 0: grid row y runs phase y / zrows over group y % zrows, its
+    // columns (yq, xq) of an image ph_w wide.
+    uint32_t phases, zrows, ph_s, ph_w;
+    FastDiv div_wp;
+    PhaseDesc ph[kMaxPhases];
 };
+
+// Column j's place in C.
+__device__ __forceinline__ float *c_column(float *c, uint32_t j, const SplitArgs &g, uint32_t py, uint32_t px) {
+    if (g.npos == 0) return c + j;
+    const uint32_t img = fdiv(j, g.div_npos), p = j - img * g.npos;
+    c += (size_t)img * g.c_img;
+    if (g.phases == 0) return c + p;
+    const uint32_t yq = fdiv(p, g.div_wp), xq = p - yq * g.div_wp.d;
+    return c + (size_t)(g.ph_s * yq + py) * g.ph_w + g.ph_s * xq + px;
+}
 
 __device__ __forceinline__ void tile_of(uint32_t w, const SplitArgs &g, uint32_t &tm, uint32_t &tn, uint32_t &split) {
     const uint32_t tiles = g.tiles_m * g.tiles_n;
@@ -247,7 +296,7 @@ struct ColLoad : ColBase<R> {
         if (span) {
             const uint32_t i0 = fdiv(r0, g.div_npos), i = fdiv(r0 + r, g.div_npos);
             base = b + (size_t)i0 * g.b_img;
-            off = 4 * ((i - i0) * g.b_img + (r0 + r - i * g.npos));
+            off = 4 * ((i - i0) * (uint32_t)g.b_img + (r0 + r - i * g.npos));
         } else {
             base = b + r0;
             off = 4 * r;
@@ -269,6 +318,247 @@ struct ColLoad : ColBase<R> {
     }
 };
 
+// fdiv without its branch on a divisor of 1.
+__device__ __forceinline__ uint32_t fdiv_select(uint32_t n, const FastDiv &f) {
+    const uint32_t one = 0u - (uint32_t)(f.mul == 0), q = umulhi32(n, f.mul) >> f.shr;
+    return (q & ~one) | (n & one);
+}
+
+// The im2col columns of a convolution, one output position a lane. The
+// position is taken apart once; the k of a load is the same in every lane of
+// the wave, so its channel and tap are scalar arithmetic. A tap outside the
+// image reads as 0: its bit in the lane's row or column mask sends the load's
+// offset past the buffer's end, where buffer loads return 0.
+template <int R>
+struct GatherLoad : ColBase<R> {
+    using ColBase<R>::kT;
+    using ColBase<R>::v;
+    using ColBase<R>::kq;
+    __amdgpu_buffer_rsrc_t buf;
+    uint32_t off;        // byte offset of the window's first tap
+    uint32_t rout, cout; // bit kh (kw) set: that row (column) of the window is outside
+    uint32_t hw;         // H * W
+
+    static __device__ __forceinline__ uint32_t outside(int first, uint32_t window, uint32_t size) {
+        const int lo = first < 0 ? -first : 0, hi = min((int)window, (int)size - first);
+        if (hi <= lo) return ~0u;
+        return ~((hi >= 32 ? ~0u : (1u << hi) - 1) & ~((1u << lo) - 1));
+    }
+    __device__ __forceinline__ void init(const float *b, const ConvGeom &cv, uint32_t r0, int tid, const SplitArgs &g) {
+        kq = __builtin_amdgcn_readfirstlane(tid / R);
+        hw = cv.H * cv.W;
+        const uint32_t r = r0 + tid % R, rr = r < g.n ? r : g.n - 1;
+        const uint32_t i0 = fdiv(r0, g.div_npos), i = fdiv(rr, g.div_npos), p = rr - i * g.npos;
+        const uint32_t h = fdiv(p, cv.div_wo), w = p - h * cv.div_wo.d;
+        rout = r < g.n ? outside((int)(h * cv.stride) - cv.pad, cv.rows, cv.H) : ~0u;
+        cout = outside((int)(w * cv.stride) - cv.pad_x, cv.cols, cv.W);
+        off = 4 * ((i - i0) * (uint32_t)g.b_img + h * cv.stride * cv.W + w * cv.stride);
+        const float *first = b + (size_t)i0 * g.b_img - ((int64_t)cv.pad * cv.W + cv.pad_x);
+        buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(first), 0, 0x80000000u, 0x00020000);
+    }
+    template <bool TAIL>
+    __device__ __forceinline__ void load_taps(const ConvGeom &cv, uint32_t k0, uint32_t kend) {
+        const uint32_t k = k0 + kq * kT;
+        const uint32_t c = fdiv_select(k, cv.div_kk), t = k - c * cv.div_kk.d;
+        uint32_t kh = fdiv_select(t, cv.div_k), kw = t - kh * cv.cols;
+        uint32_t at = 4 * (c * hw + kh * cv.W + kw);
+        const uint32_t next_row = 4 * (cv.W - cv.cols), next_chan = 4 * (hw - cv.rows * cv.W);
+#pragma unroll
+        for (int j = 0; j < kT; ++j) {
+            if (!TAIL || k + j < kend) {
+                const uint32_t out = (uint32_t)(__builtin_amdgcn_sbfe((int)rout, kh, 1) | __builtin_amdgcn_sbfe((int)cout, kw, 1));
+                v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(buf, off | out, at, 0));
+            } else {
+                v[j] = 0.0f;
+            }
+            // The next tap, without branches (the loads stay in one basic block).
+            const uint32_t row = 0u - (uint32_t)(kw + 1 == cv.cols);
+            const uint32_t chan = row & (0u - (uint32_t)(kh + 1 == cv.rows));
+            kw = (kw + 1) & ~row;
+            kh = (kh - row) & ~chan;
+            at += 4 + (row & next_row) + (chan & next_chan);
+        }
+    }
+    __device__ __forceinline__ void load(uint32_t k0, const ConvGeom &cv) { load_taps<false>(cv, k0, 0); }
+    __device__ __forceinline__ void load_tail(uint32_t k0, uint32_t kend, const ConvGeom &cv) { load_taps<true>(cv, k0, kend); }
+};
+
+// The same with 64-bit addresses and compared bounds.
+template <int R>
+struct GatherWideLoad : ColBase<R> {
+    using ColBase<R>::kT;
+    using ColBase<R>::v;
+    using ColBase<R>::kq;
+    const float *img;
+    int y, x;
+    bool in;
+
+    __device__ __forceinline__ void init(const float *b, const ConvGeom &cv, uint32_t r0, int tid, const SplitArgs &g) {
+        kq = __builtin_amdgcn_readfirstlane(tid / R);
+        const uint32_t r = r0 + tid % R, rr = r < g.n ? r : g.n - 1;
+        const uint32_t i = fdiv(rr, g.div_npos), p = rr - i * g.npos;
+        const uint32_t h = fdiv(p, cv.div_wo), w = p - h * cv.div_wo.d;
+        in = r < g.n;
+        y = (int)(h * cv.stride) - cv.pad;
+        x = (int)(w * cv.stride) - cv.pad_x;
+        img = b + (size_t)i * g.b_img;
+    }
+    __device__ __forceinline__ void load_tail(uint32_t k0, uint32_t kend, const ConvGeom &cv) {
+#pragma unroll
+        for (int j = 0; j < kT; ++j) {
+            const uint32_t k = k0 + kq * kT + j;
+            const uint32_t c = fdiv(k, cv.div_kk), t = k - c * cv.div_kk.d;
+            const uint32_t kh = fdiv(t, cv.div_k), kw = t - kh * cv.cols;
+            const int yy = y + (int)kh, xx = x + (int)kw;
+            const bool ok = in && k < kend && yy >= 0 && yy < (int)cv.H && xx >= 0 && xx < (int)cv.W;
+            v[j] = ok ? img[((size_t)c * cv.H + yy) * cv.W + xx] : 0.0f;
+        }
+    }
+    __device__ __forceinline__ void load(uint32_t k0, const ConvGeom &cv) { load_tail(k0, ~0u, cv); }
+};
+
+// The quad of k at k0 + 4 * (tid % 4) of a weight gradient: its image (from the
+// split's first one on) and first position; `in` says whether it is there. The
+// host gives the kernels that use it images, positions and image sides below
+// 2^24, so that all products but those with the image stride are 24-bit ones.
+struct Quad {
+    uint32_t img, p;
+    bool in;
+    __device__ __forceinline__ Quad(uint32_t k0, uint32_t kend, uint32_t img0, int tid, const SplitArgs &g) {
+        const uint32_t k = k0 + 4 * (tid % 4);
+        const uint32_t i = fdiv_select(k, g.div_kpos4);
+        in = k < kend;
+        img = i - img0;
+        p = k - __umul24(i, g.div_kpos4.d);
+    }
+};
+
+// Where the four floats of thread tid's float4 l of a slab go: as RowLoad's.
+template <int R>
+struct QuadBase {
+    static constexpr int kL = RowLoad<R>::kL;
+    RowLoad<R> row;  // v and mx only
+    __device__ __forceinline__ void store(uint32_t *s, int tid) { row.store(s, tid); }
+    __device__ __forceinline__ void store_f32(float *s, int tid) const { row.store_f32(s, tid); }
+    __device__ __forceinline__ bool tiny() const { return row.tiny(); }
+};
+
+// Rows of delta (row stride kpos): four positions in one 16-byte load. ODD: an
+// image's last quad has fewer; it is loaded from kpos - 4 and shifted.
+template <int R, bool ODD>
+struct SegLoad : QuadBase<R> {
+    using QuadBase<R>::kL;
+    using QuadBase<R>::row;
+    __amdgpu_buffer_rsrc_t buf;
+    uint32_t at[kL], img0;
+
+    __device__ __forceinline__ void init(const float *base, uint32_t r0, uint32_t rows, uint32_t kbeg, int tid,
+                                         uint64_t img_stride, const SplitArgs &g) {
+        img0 = fdiv_select(kbeg, g.div_kpos4);
+#pragma unroll
+        for (int l = 0; l < kL; ++l) {
+            const uint32_t f = tid + l * kBlock, r = f / 4 < rows ? f / 4 : rows - 1;
+            at[l] = 4 * r * g.kpos;
+        }
+        buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + (size_t)img0 * img_stride + (size_t)r0 * g.kpos), 0,
+                                                0x80000000u, 0x00020000);
+    }
+    __device__ __forceinline__ void load(uint32_t k0, uint32_t kend, int tid, uint64_t img_stride, const SplitArgs &g) {
+        const Quad q(k0, kend, img0, tid, g);
+        const uint32_t p = ODD ? min(q.p, g.kpos - 4) : q.p, d = q.p - p;
+        const uint32_t off = 4 * (q.img * (uint32_t)img_stride + p);
+#pragma unroll
+        for (int l = 0; l < kL; ++l) {
+            const auto t = __builtin_amdgcn_raw_buffer_load_b128(buf, (off + at[l]) | (q.in ? 0u : 0x80000000u), 0, 0);
+            float4 v = make_float4(__uint_as_float(t[0]), __uint_as_float(t[1]), __uint_as_float(t[2]), __uint_as_float(t[3]));
+            if constexpr (ODD) {
+                if (d & 1) v = make_float4(v.y, v.z, v.w, 0.0f);
+                if (d & 2) v = make_float4(v.z, v.w, 0.0f, 0.0f);
+            }
+            row.v[l] = v;
+        }
+    }
+};
+
+// Rows of the input's im2col: one tap of one channel a row (fixed for the
+// thread), its element at each position of the quad.
+template <int R>
+struct TapLoad : QuadBase<R> {
+    using QuadBase<R>::kL;
+    using QuadBase<R>::row;
+    __amdgpu_buffer_rsrc_t buf;
+    uint32_t img0;
+    int at[kL], dy[kL], dx[kL];
+
+    __device__ __forceinline__ void init(const float *base, const ConvGeom &cv, uint32_t r0, uint32_t rows, uint32_t kbeg,
+                                         int tid, const SplitArgs &g) {
+        img0 = fdiv_select(kbeg, g.div_kpos4);
+#pragma unroll
+        for (int l = 0; l < kL; ++l) {
+            const uint32_t f = tid + l * kBlock, r = r0 + (f / 4 < rows ? f / 4 : rows - 1);
+            const uint32_t c = fdiv_select(r, cv.div_kk), t = r - c * cv.div_kk.d;
+            const uint32_t kh = fdiv_select(t, cv.div_k);
+            dy[l] = (int)kh - cv.pad;
+            dx[l] = (int)(t - kh * cv.cols) - cv.pad_x;
+            at[l] = (int)(c * cv.H * cv.W) + dy[l] * (int)cv.W + dx[l];
+        }
+        buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + (size_t)img0 * g.b_img), 0, 0x80000000u, 0x00020000);
+    }
+    __device__ __forceinline__ void load(uint32_t k0, uint32_t kend, int tid, const ConvGeom &cv, const SplitArgs &g) {
+        const Quad q(k0, kend, img0, tid, g);
+        const uint32_t h = fdiv_select(q.p, cv.div_wo), last = __umul24(cv.div_wo.d - 1, cv.stride);
+        uint32_t y = __umul24(h, cv.stride), x = __umul24(q.p - __umul24(h, cv.div_wo.d), cv.stride);
+        uint32_t pos = q.img * (uint32_t)g.b_img + __umul24(y, cv.W) + x;
+        const uint32_t wrap_pos = cv.stride * cv.W - last;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const bool in = q.in & (q.p + j < g.kpos);
+#pragma unroll
+            for (int l = 0; l < kL; ++l) {
+                // Unsigned: below 0 is out too. No branches (see the step's one basic block).
+                const bool ok = in & (y + dy[l] < cv.H) & (x + dx[l] < cv.W);
+                ::dkz::lane(row.v[l], j) =
+                    __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(buf, 4 * (pos + at[l]) | (ok ? 0u : 0x80000000u), 0, 0));
+            }
+            const bool wrap = x == last;
+            x = wrap ? 0 : x + cv.stride;
+            y += wrap ? cv.stride : 0;
+            pos += wrap ? wrap_pos : cv.stride;
+        }
+    }
+};
+
+// Both with 64-bit addresses: img + r * kpos + p, and the tap's element.
+template <int R, bool TAP>
+struct QuadWideLoad : QuadBase<R> {
+    using QuadBase<R>::kL;
+    using QuadBase<R>::row;
+    __device__ __forceinline__ void load(const float *base, uint32_t r0, uint32_t rows, uint32_t k0, uint32_t kend, int tid,
+                                         uint64_t img_stride, const ConvGeom &cv, const SplitArgs &g) {
+        const Quad q(k0, kend, 0, tid, g);
+#pragma unroll
+        for (int l = 0; l < kL; ++l) {
+            const uint32_t f = tid + l * kBlock, r = r0 + (f / 4 < rows ? f / 4 : rows - 1);
+            const uint32_t c = fdiv(r, cv.div_kk), t = r - c * cv.div_kk.d, kh = fdiv(t, cv.div_k), kw = t - kh * cv.cols;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t p = q.p + j;
+                bool ok = q.in && p < g.kpos;
+                size_t e = (size_t)q.img * img_stride;
+                if constexpr (TAP) {
+                    const uint32_t h = fdiv(p, cv.div_wo), w = p - h * cv.div_wo.d;
+                    const int y = (int)(h * cv.stride + kh) - cv.pad, x = (int)(w * cv.stride + kw) - cv.pad_x;
+                    ok = ok && y >= 0 && y < (int)cv.H && x >= 0 && x < (int)cv.W;
+                    e += ((size_t)c * cv.H + y) * cv.W + x;
+                } else {
+                    e += (size_t)r * g.kpos + p;
+                }
+                ::dkz::lane(row.v[l], j) = ok ? base[e] : 0.0f;
+            }
+        }
+    }
+};
+
 // C(i, j) = beta-applied C + alpha * s (gemm.zig:121-131: beta == 0 clears C,
 // NaN included).
 __device__ __forceinline__ float gemm_out(const float *cp, float s, float alpha, float beta) {
@@ -276,6 +566,18 @@ __device__ __forceinline__ float gemm_out(const float *cp, float s, float alpha,
     if (beta != 0.0f) cv = (beta == 1.0f) ? *cp : *cp * beta;
     return cv + alpha * s;
 }
+
+template <Operand K, int R>
+struct Loader;
+template <int R> struct Loader<kRowMajor, R> { using type = RowLoad<R>; };
+template <int R> struct Loader<kColMajor, R> { using type = ColLoad<R>; };
+template <int R> struct Loader<kGather, R> { using type = GatherLoad<R>; };
+template <int R> struct Loader<kGatherWide, R> { using type = GatherWideLoad<R>; };
+template <int R> struct Loader<kSeg, R> { using type = SegLoad<R, false>; };
+template <int R> struct Loader<kSegOdd, R> { using type = SegLoad<R, true>; };
+template <int R> struct Loader<kTap, R> { using type = TapLoad<R>; };
+template <int R> struct Loader<kSegWide, R> { using type = QuadWideLoad<R, false>; };
+template <int R> struct Loader<kTapWide, R> { using type = QuadWideLoad<R, true>; };
 
 // Interleaves a step's VALU work with its MFMAs (each occupies the matrix core
 // for the time of eight VALU instructions).
@@ -299,43 +601,88 @@ constexpr int min_waves() { return BM * BN >= 128 * 128 ? 2 : BM * BN >= 128 * 6
 
 template <int BM, int BN, Operand AK, Operand BK>
 __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kernel(SplitArgs g) {
-    constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-    constexpr int kA = slab_words<BM>(), kB = slab_words<BN>();
+    constexpr int kRowsOfWaves = BM == 32 ? 1 : 2;  // 32-row tiles: four waves side by side
+    constexpr int WM = BM / kRowsOfWaves, WN = BN * kRowsOfWaves / 4, TM = WM / 32, TN = WN / 32;
+    constexpr int RA = BM == 32 ? 64 : BM;  // rows of A staged (of a 32-row tile, the last row again)
+    constexpr int kA = slab_words<RA>(), kB = slab_words<BN>();
     __shared__ __align__(16) uint32_t lds[2 * (kA + kB)];
-    static_assert((BM + BN) * kF32Pitch <= 2 * (kA + kB), "the fp32 pass uses the same LDS");
+    static_assert((RA + BN) * kF32Pitch <= 2 * (kA + kB), "the fp32 pass uses the same LDS");
 
-    const uint32_t z = blockIdx.y;
+    constexpr bool kGa = BK == kGather || BK == kGatherWide;
+    constexpr bool kQuads = AK >= kSeg;  // a weight gradient: quads past kend load as zeros
+    uint32_t z = blockIdx.y;
+    // A phase's row of a strided data gradient takes its taps, window and
+    // pixel offsets (fields picked with constant indexes, so the arguments
+    // stay where they are).
+    const float *a_base = g.a;
+    uint32_t k_all = g.k, k_chunk = g.k_chunk, lda = g.lda, py = 0, px = 0;
+    uint64_t a_z = g.a_z;
+    ConvGeom cv = g.cv;
+    if (kGa && g.phases != 0) {
+        const uint32_t p = z / g.zrows;
+        z -= p * g.zrows;
+#define DKZ_PHASE_FIELD(f) (p == 0 ? g.ph[0].f : p == 1 ? g.ph[1].f : p == 2 ? g.ph[2].f : g.ph[3].f)
+        a_base = DKZ_PHASE_FIELD(a);
+        k_all = DKZ_PHASE_FIELD(k);
+        cv.rows = DKZ_PHASE_FIELD(rows);
+        cv.cols = DKZ_PHASE_FIELD(cols);
+        cv.pad = DKZ_PHASE_FIELD(pad);
+        cv.pad_x = DKZ_PHASE_FIELD(pad_x);
+        cv.div_kk = DKZ_PHASE_FIELD(div_kk);
+        cv.div_k = DKZ_PHASE_FIELD(div_k);
+        py = DKZ_PHASE_FIELD(py);
+        px = DKZ_PHASE_FIELD(px);
+#undef DKZ_PHASE_FIELD
+        k_chunk = lda = k_all;
+        a_z = (uint64_t)g.m * k_all;
+    }
     uint32_t tm, tn, split;
     tile_of(blockIdx.x, g, tm, tn, split);
-    const float *ga = g.a + (size_t)(z % g.zgroups) * g.a_z;
+    const float *ga = a_base + (size_t)(z % g.zgroups) * a_z;
     const float *gb = g.b + (size_t)z * g.b_z;
     float *gc = g.c + (size_t)z * g.c_z;
     const uint32_t m0 = tm * BM, n0 = tn * BN;
-    const uint32_t kbeg = split * g.k_chunk;
-    const uint32_t kend = kbeg + g.k_chunk < g.k ? kbeg + g.k_chunk : g.k;
+    const uint32_t kbeg = split * k_chunk;
+    const uint32_t kend = kbeg + k_chunk < k_all ? kbeg + k_chunk : k_all;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm0 = (wave >> 1) * WM, wn0 = (wave & 1) * WN;
+    const int wm0 = BM == 32 ? 0 : (wave >> 1) * WM, wn0 = (BM == 32 ? wave : wave & 1) * WN;
     const int half = lane >> 5, l32 = lane & 31;
 
-    std::conditional_t<AK == kRowMajor, RowLoad<BM>, ColLoad<BM>> sa[2];
-    std::conditional_t<BK == kRowMajor, RowLoad<BN>, ColLoad<BN>> sb[2];
     // Two register sets: slab s is loaded into set s & 1.
+    typename Loader<AK, RA>::type sa[2];
+    typename Loader<BK, BN>::type sb[2];
+    const uint32_t rows_a = BM == 32 ? min(g.m - m0, 32u) : g.m - m0, rows_b = g.n - n0;
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
-        if constexpr (AK == kRowMajor) sa[d].init(ga, g.lda, m0, g.m - m0, tid);
-        else sa[d].init(ga, g.lda, m0, g.m - m0, tid, g, false);
-        if constexpr (BK == kRowMajor) sb[d].init(gb, g.ldb, n0, g.n - n0, tid);
-        else sb[d].init(gb, g.ldb, n0, g.n - n0, tid, g, g.npos != 0);
+        if constexpr (AK == kRowMajor) sa[d].init(ga, lda, m0, rows_a, tid);
+        else if constexpr (AK == kColMajor) sa[d].init(ga, lda, m0, rows_a, tid, g, false);
+        else if constexpr (AK == kSeg || AK == kSegOdd) sa[d].init(ga, m0, rows_a, kbeg, tid, g.a_img, g);
+        if constexpr (BK == kRowMajor) sb[d].init(gb, g.ldb, n0, rows_b, tid);
+        else if constexpr (BK == kColMajor) sb[d].init(gb, g.ldb, n0, rows_b, tid, g, g.npos != 0);
+        else if constexpr (kGa) sb[d].init(gb, cv, n0, tid, g);
+        else if constexpr (BK == kSeg || BK == kSegOdd) sb[d].init(gb, n0, rows_b, kbeg, tid, g.b_img, g);
+        else if constexpr (BK == kTap) sb[d].init(gb, cv, n0, rows_b, kbeg, tid, g);
     }
     auto load = [&](int d, uint32_t k0) {
-        sa[d].load(k0);
-        sb[d].load(k0);
+        if constexpr (AK == kSeg || AK == kSegOdd) sa[d].load(k0, kend, tid, g.a_img, g);
+        else if constexpr (AK == kSegWide) sa[d].load(ga, m0, rows_a, k0, kend, tid, g.a_img, cv, g);
+        else sa[d].load(k0);
+        if constexpr (kGa) sb[d].load(k0, cv);
+        else if constexpr (BK == kSeg || BK == kSegOdd) sb[d].load(k0, kend, tid, g.b_img, g);
+        else if constexpr (BK == kTap) sb[d].load(k0, kend, tid, cv, g);
+        else if constexpr (BK == kTapWide) sb[d].load(gb, n0, rows_b, k0, kend, tid, g.b_img, cv, g);
+        else sb[d].load(k0);
     };
-    auto load_tail = [&](uint32_t k0) {
-        if constexpr (AK == kRowMajor) sa[0].load_tail(k0, kend, tid);
-        else sa[0].load_tail(k0, kend);
-        if constexpr (BK == kRowMajor) sb[0].load_tail(k0, kend, tid);
-        else sb[0].load_tail(k0, kend);
+    auto load_tail = [&](int d, uint32_t k0) {
+        if constexpr (kQuads) {
+            load(d, k0);
+        } else {
+            if constexpr (AK == kRowMajor) sa[d].load_tail(k0, kend, tid);
+            else sa[d].load_tail(k0, kend);
+            if constexpr (BK == kRowMajor) sb[d].load_tail(k0, kend, tid);
+            else if constexpr (kGa) sb[d].load_tail(k0, kend, cv);
+            else sb[d].load_tail(k0, kend);
+        }
     };
     auto store = [&](int d) {  // set d to LDS buffer d
         uint32_t *to = lds + d * (kA + kB);
@@ -353,13 +700,13 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
 
     auto compute = [&](int cur) {
         bf16x8 af[TM][kPlanes], bf[TN][kPlanes];
-        const uint32_t *pa = lds + cur * (kA + kB) + half * half_words<BM>() + (wm0 + l32) * 4;
+        const uint32_t *pa = lds + cur * (kA + kB) + half * half_words<RA>() + (wm0 + l32) * 4;
         const uint32_t *pb = lds + cur * (kA + kB) + kA + half * half_words<BN>() + (wn0 + l32) * 4;
 #pragma unroll
         for (int u = 0; u < kPlanes; ++u) {
 #pragma unroll
             for (int ti = 0; ti < TM; ++ti)
-                af[ti][u] = *reinterpret_cast<const bf16x8 *>(pa + u * 2 * half_words<BM>() + ti * 128);
+                af[ti][u] = *reinterpret_cast<const bf16x8 *>(pa + u * 2 * half_words<RA>() + ti * 128);
 #pragma unroll
             for (int tj = 0; tj < TN; ++tj)
                 bf[tj][u] = *reinterpret_cast<const bf16x8 *>(pb + u * 2 * half_words<BN>() + tj * 128);
@@ -381,8 +728,8 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
     // s + 1 and loads slab s + 3 into the registers that held it (past the last
     // slab the last one again, unused): one basic block whose VALU work the
     // scheduler is told to place between the MFMAs.
-    const uint32_t whole = kend > kbeg ? (kend - kbeg) / kBK : 0;
-    const bool tail = kend > kbeg && (kend - kbeg) % kBK != 0;
+    const uint32_t whole = kend > kbeg ? (kend - kbeg + (kQuads ? kBK - 1 : 0)) / kBK : 0;
+    const bool tail = !kQuads && kend > kbeg && (kend - kbeg) % kBK != 0;
     if (whole > 0) {
         const auto slab_k = [&](uint32_t x) { return kbeg + (x < whole ? x : whole - 1) * kBK; };
         const auto step = [&](auto d, uint32_t s) {
@@ -394,7 +741,8 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
             __syncthreads();
         };
         load(0, slab_k(0));
-        load(1, slab_k(1));
+        if (tail && whole == 1) load_tail(1, kbeg + kBK);  // a first layer's 27 k: both slabs at once
+        else load(1, slab_k(1));
         store(0);
         load(0, slab_k(2));
         __syncthreads();
@@ -410,10 +758,14 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
         }
     }
     if (tail) {
-        load_tail(kbeg + whole * kBK);
-        store(0);
+        if (whole == 1) {
+            store(1);
+        } else {
+            load_tail(0, kbeg + whole * kBK);
+            store(0);
+        }
         __syncthreads();
-        compute(0);
+        compute(whole == 1);
         __syncthreads();
     }
 
@@ -429,7 +781,7 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
             for (int r = 0; r < 16; ++r) redo |= !(fabsf(big[ti][tj][r]) < __builtin_inff());
         }
     if (__syncthreads_or(redo)) {
-        float *as = reinterpret_cast<float *>(lds), *bs = as + BM * kF32Pitch;
+        float *as = reinterpret_cast<float *>(lds), *bs = as + RA * kF32Pitch;
 #pragma unroll
         for (int ti = 0; ti < TM; ++ti)
 #pragma unroll
@@ -439,7 +791,7 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
 #pragma unroll 1
         for (uint32_t k0 = kbeg; k0 < kend; k0 += kBK) {
             if (k0 + kBK <= kend) load(0, k0);
-            else load_tail(k0);
+            else load_tail(0, k0);
             sa[0].store_f32(as, tid);
             sb[0].store_f32(bs, tid);
             __syncthreads();
@@ -457,30 +809,73 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
     }
 
     // big[ti][tj][r] is C(row, col) of the wave's block (ti, tj) with
-    // row = 8*(r/4) + 4*(lane/32) + r%4 and col = lane%32.
+    // row = 8*(r/4) + 4*(lane/32) + r%4 and col = lane%32. A block's sixteen
+    // values of C are loaded together (rows past m read row m - 1), then stored.
 #pragma unroll
     for (int tj = 0; tj < TN; ++tj) {
         const uint32_t j = n0 + wn0 + tj * 32 + l32;
         if (j >= g.n) continue;
-        float *ccol = gc + j;
-        if (g.npos != 0) {
-            const uint32_t img = fdiv(j, g.div_npos);
-            ccol = gc + (size_t)img * g.c_img + (j - img * g.npos);
-        }
+        float *ccol = c_column(gc, j, g, py, px);
 #pragma unroll
-        for (int ti = 0; ti < TM; ++ti)
+        for (int ti = 0; ti < TM; ++ti) {
+            const uint32_t i0 = m0 + wm0 + ti * 32 + half * 4;
+            const auto row = [&](int r) { return i0 + (r >> 2) * 8 + (r & 3); };
+            float *to = g.splits > 1 ? g.partial + (size_t)split * g.m * g.n + j : ccol;
+            const uint32_t ld = g.splits > 1 ? g.n : g.ldc;
+            float out[16];
+            if (g.splits > 1) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t i = m0 + wm0 + ti * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
-                if (i >= g.m) continue;
-                if (g.splits > 1) {
-                    g.partial[((size_t)split * g.m + i) * g.n + j] = big[ti][tj][r];
-                } else {
-                    float *cp = ccol + (size_t)i * g.ldc;
-                    *cp = gemm_out(cp, big[ti][tj][r], g.alpha, g.beta);
-                }
+                for (int r = 0; r < 16; ++r) out[r] = big[ti][tj][r];
+            } else if (g.beta == 0.0f) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) out[r] = 0.0f + g.alpha * big[ti][tj][r];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) out[r] = to[(size_t)min(row(r), g.m - 1) * ld];
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    out[r] = (g.beta == 1.0f ? out[r] : out[r] * g.beta) + g.alpha * big[ti][tj][r];
             }
+            if (m0 + BM <= g.m) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) to[(size_t)row(r) * ld] = out[r];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (row(r) < g.m) to[(size_t)row(r) * ld] = out[r];
+            }
+        }
     }
+}
+
+// The split-K epilogue: adds a tile's partials in split order, then as the
+// kernel's own epilogue. V4: a lane takes four consecutive columns of one row
+// (one image's, 16-byte aligned).
+template <bool V4, int kReduceBatch>
+__global__ __launch_bounds__(kBlock) void split_reduce_kernel(SplitArgs g) {
+    using T = std::conditional_t<V4, float4, float>;
+    constexpr uint32_t kW = V4 ? 4 : 1;
+    const uint32_t mn = g.m * g.n, v = blockIdx.x * kBlock + threadIdx.x;
+    if (v >= mn / kW) return;
+    const uint32_t e = v * kW, i = e / g.n, j = e - i * g.n;
+    // kReduceBatch partials in flight at a time; the missing ones of the last batch
+    // are +0, which leaves the sum as is.
+    float s[kW] = {};
+    for (uint32_t t = 0; t < g.splits; t += kReduceBatch) {
+        T p[kReduceBatch];
+#pragma unroll
+        for (int u = 0; u < kReduceBatch; ++u)
+            p[u] = t + u < g.splits ? reinterpret_cast<const T *>(g.partial + (size_t)(t + u) * mn)[v] : T{};
+#pragma unroll
+        for (int u = 0; u < kReduceBatch; ++u)
+#pragma unroll
+            for (uint32_t x = 0; x < kW; ++x) s[x] += reinterpret_cast<const float *>(&p[u])[x];
+    }
+    float *cp = c_column(g.c, j, g, 0, 0) + (size_t)i * g.ldc;
+    T o;
+#pragma unroll
+    for (uint32_t x = 0; x < kW; ++x) reinterpret_cast<float *>(&o)[x] = gemm_out(cp + x, s[x], g.alpha, g.beta);
+    *reinterpret_cast<T *>(cp) = o;
 }
 
 }  // namespace

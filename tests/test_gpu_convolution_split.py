@@ -1,0 +1,82 @@
+"""The convolution entry points where their product kernel's tiles, slabs and
+operand loaders end: 32-row tiles, 27 k (one whole slab of 16 and a tail), K in
+several ranges, windows over 32 wide (64-bit gathers), one to three positions an
+image (64-bit weight-gradient loads), positions that are no multiple of four,
+many images in one tile -- and infinities and NaNs, which take the fp32 matrix
+instruction. References and tolerances are test_gpu_convolution's."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from darknet_zig_amd import gpu
+from oracle import ref
+from tests import test_gpu_convolution as base
+from tests.helpers import down, rng, up
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # batch, groups, channels, height, width, filters, ksize, stride, pad
+    (2, 1, 3, 33, 31, 20, 3, 1, 1),    # 27 k, a 32-row tile
+    (8, 1, 3, 40, 40, 32, 3, 2, 1),    # the same, stride 2
+    (1, 1, 512, 13, 13, 96, 3, 1, 1),  # one small image: K in ranges
+    (2, 2, 64, 9, 9, 72, 3, 1, 1),     # two groups: K whole
+    (2, 1, 2, 36, 36, 4, 33, 1, 2),    # a window of 33
+    (2, 1, 4, 35, 70, 6, 34, 33, 1),   # the same with stride 33
+    (2, 1, 4, 21, 19, 6, 7, 2, 3),
+    (3, 1, 5, 1, 1, 4, 1, 1, 0),       # one position an image
+    (7, 1, 4, 3, 1, 5, 3, 1, 1),       # three
+    (9, 1, 6, 2, 2, 33, 1, 1, 0),      # four
+    (300, 1, 3, 3, 3, 130, 3, 1, 1),   # fourteen images in a column tile
+    (40, 1, 20, 13, 13, 33, 3, 1, 1),
+    (3, 1, 140, 5, 7, 130, 1, 1, 0),   # 35 positions, ksize 1
+    (1, 1, 7, 40, 50, 129, 1, 1, 0),
+    (2, 1, 130, 24, 24, 128, 3, 2, 1),  # four phases of 144 positions
+]
+
+
+@pytest.mark.parametrize("case", SHAPES, ids=str)
+def test_forward(dev, case):
+    base.test_convolution_forward(dev, case)
+
+
+@pytest.mark.parametrize("case", SHAPES, ids=str)
+def test_weight_gradient(dev, case):
+    base.test_convolution_weight_gradient(dev, case)
+
+
+@pytest.mark.parametrize("case", SHAPES, ids=str)
+def test_data_gradient(dev, case):
+    base.test_convolution_data_gradient(dev, case)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("case", [(2, 1, 8, 9, 9, 40, 3, 1, 1), (2, 1, 8, 8, 8, 40, 1, 1, 0)], ids=str)
+def test_values_that_are_not_finite(dev, case, value):
+    """One such element of the input: the outputs and weight updates it
+    reaches are what IEEE arithmetic makes them, the others within the bound."""
+    batch, groups, C, H, W, F, ks, s, p = case
+    r = rng(3)
+    x = r.uniform(-1, 1, batch * C * H * W).astype(np.float32)
+    x[C * H * W + 3 * H * W + 4 * W + 5] = value
+    w = r.uniform(0.1, 1, F * C * ks * ks).astype(np.float32)
+    n = ref.conv_out_dim(H, ks, s, p) * ref.conv_out_dim(W, ks, s, p)
+    d = r.uniform(0.1, 1, batch * F * n).astype(np.float32)
+    with np.errstate(all="ignore"):
+        fwd = base._reference(case, x, w, np.zeros(batch * F * n, np.float32))[:2]
+        wgr = base._wgrad_reference(case, x, d, np.zeros(w.size, np.float32))
+    dx, dw, dd = up(x), up(w), up(d)
+    out, upd = gpu.alloc(d.size), gpu.alloc(w.size)
+    gpu.convolutionForward(batch, groups, C, H, W, F, ks, s, p, dw, dx, out)
+    gpu.convolutionWeightGradient(batch, groups, C, H, W, F, ks, s, p, dd, dx, upd)
+    for got, (want, bd) in ((down(out, d), fwd), (down(upd, w), wgr)):
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        inf = np.isinf(want)
+        assert np.array_equal(got[inf], want[inf].astype(np.float32))
+        fin = np.isfinite(want)
+        assert fin.any() and not fin.all()
+        assert np.all(np.abs(got[fin] - want[fin]) <= bd[fin])
+    for b in (dx, dw, dd, out, upd):
+        gpu.free(b)
