@@ -38,28 +38,21 @@
 // (blas.zig:121-135) sums f32-rounded (x - m)^2 terms sequentially in f32, so
 // the two agree to within the twin's own rounding error.
 //
-// The fast path needs spatial % 4 == 0, 16-byte aligned tensors and a
-// non-empty tensor; any other call runs the per-op sequence, which handles
-// every shape (and edge case) exactly as the individual entry points do.
+// These passes need spatial % 4 == 0 and 16-byte aligned tensors; other
+// tensors take batchnorm_ragged.hip's passes, and empty ones (and the few
+// those leave) the per-op sequence, which handles every shape (and edge
+// case) exactly as the individual entry points do.
 #include <atomic>
 #include <cstdlib>
 #include <type_traits>
 
-#include "dkz_channel.hpp"
+#include "bn_common.hpp"
 #include "dkz_hints.hpp"
 
 namespace dkz {
 namespace {
 
 constexpr int kUnroll = 4;
-constexpr float kMomentum = 0.99f;          // rolling_momentum, batchnorm.zig:16 (f32)
-constexpr float kAlpha = 1.0f - kMomentum;  // batchnorm.zig:141: an f32 subtraction, exact
-
-template <int NS>
-struct Sums {
-    double s[NS];
-};
-
 // f(std::integral_constant<int, I>) for I = B, B + S, ... < E: a loop whose
 // index is a compile-time constant in each step (so arrays indexed by it
 // stay in registers, however long the body).
@@ -110,95 +103,7 @@ __device__ __forceinline__ void red_coords(const RedGeom &g, uint32_t &f, uint32
     }
 }
 
-// NS sums over a BS-thread workgroup; the result is valid in wave 0. Each
-// wave's sums go through LDS (lds holds NS * BS/64 doubles) and wave 0 adds
-// them with one more DPP reduction, so the order is fixed by the shape.
-template <int NS, int BS>
-__device__ __forceinline__ Sums<NS> block_sums(const double (&a)[NS], double *lds) {
-    constexpr int W = BS / kWave;
-    const int w = threadIdx.x / kWave, l = threadIdx.x & (kWave - 1);
-    Sums<NS> r;
-#pragma unroll
-    for (int q = 0; q < NS; ++q) {
-        const double v = wave_sum(a[q]);
-        if (l == 0) lds[q * W + w] = v;
-    }
-    __syncthreads();
-    if (w == 0) {
-#pragma unroll
-        for (int q = 0; q < NS; ++q) r.s[q] = wave_sum(l < W ? lds[q * W + l] : 0.0);
-    }
-    return r;
-}
-
-// Partial sums of workgroup (f, k) go to partials[(q*F + f)*K + k].
-template <int NS, int BS>
-__device__ __forceinline__ void store_partials(const Sums<NS> &r, const RedGeom &g, uint32_t f, uint32_t k,
-                                               double *partials) {
-    if (threadIdx.x == 0) {
-        const uint32_t F = g.div_filters.d;
-#pragma unroll
-        for (int q = 0; q < NS; ++q) partials[((uint32_t)q * F + f) * g.K + k] = r.s[q];
-    }
-}
-
-// Second launch: one wave per channel adds its K partials of each sum in
-// index order, then finalises.
-template <int NS, class Fin>
-__global__ __launch_bounds__(kBlock) void bn_finalize_kernel(Fin fin, const double *partials, uint32_t F,
-                                                             uint32_t K) {
-    const uint32_t f = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-    if (f >= F) return;  // whole waves leave together
-    const uint32_t l = threadIdx.x & (kWave - 1);
-    Sums<NS> r;
-#pragma unroll
-    for (int q = 0; q < NS; ++q) {
-        const double *p = partials + ((uint64_t)q * F + f) * K;
-        double s = 0.0;
-        for (uint32_t i = l; i < K; i += kWave) s += p[i];
-        r.s[q] = wave_sum(s);
-    }
-    if (l == 0) fin(f, r);
-}
-
 // ---- forward ----------------------------------------------------------------
-
-// mean, variance and the rolling averages of channel f from s1 = sum(x - c),
-// s2 = sum((x - c)^2) over its n elements, c = the channel's first element.
-// The split statistics pass stores c beside the partials (shift[f]): the
-// apply pass may overwrite the input in place before every workgroup has
-// finalised.
-struct FwdFin {
-    const double *shift;
-    float *mean, *variance, *rolling_mean, *rolling_variance;
-    double n;
-    float mean_scale;  // 1/(B*S) in f32 (blas.zig:107)
-    float var_scale;   // 1/(B*S - 1) in f32 (blas.zig:122)
-    __device__ void stats(const Sums<2> &r, double c, float &m, float &v) const {
-        const double s1 = r.s[0], s2 = r.s[1];
-        m = (float)(n * c + s1) * mean_scale;  // blas.zig:114: sum * (1/(B*S))
-        const double dm = (c + s1 / n) - (double)m;
-        double m2 = s2 - s1 * (s1 / n);
-        m2 = m2 > 0.0 ? m2 : 0.0;
-        v = (float)(m2 + n * dm * dm) * var_scale;  // blas.zig:133
-    }
-    // met == false (a one-launch pass whose channel barrier gave up): the
-    // batch statistics are written (NaN) but the rolling averages, which
-    // carry over to the next call, are left as they were.
-    __device__ void write(uint32_t f, float m, float v, bool met = true) const {
-        mean[f] = m;
-        variance[f] = v;
-        if (!met) return;
-        // batchnorm.zig:140-143: scal(0.99) then axpy(1 - 0.99) -- axpy is an fma (blas.zig:22)
-        rolling_mean[f] = __builtin_fmaf(kAlpha, m, rolling_mean[f] * kMomentum);
-        rolling_variance[f] = __builtin_fmaf(kAlpha, v, rolling_variance[f] * kMomentum);
-    }
-    __device__ void operator()(uint32_t f, const Sums<2> &r) const {  // after a split pass
-        float m, v;
-        stats(r, shift[f], m, v);
-        write(f, m, v);
-    }
-};
 
 __device__ __forceinline__ void acc_shifted(float4 v, double c, double &a1, double &a2) {
     const double d0 = (double)v.x - c, d1 = (double)v.y - c, d2 = (double)v.z - c, d3 = (double)v.w - c;
@@ -242,19 +147,6 @@ __global__ __launch_bounds__(BS) void bn_stats_kernel(const float *input, RedGeo
         store_partials<2, BS>(r, g, f, k, partials);
         if (k == 0 && threadIdx.x == 0) partials[2u * g.div_filters.d * g.K + f] = c;  // = fin.shift[f]
     }
-}
-
-struct FwdParams {
-    const float *mean, *variance, *scales, *biases;
-};
-
-// What the forward apply pass needs of channel f.
-struct FwdChan {
-    float m, inv, gam, bet;
-};
-
-__device__ __forceinline__ FwdChan fwd_chan(float m, float v, float gam, float bet) {
-    return {m, 1.0f / (sqrtf(v) + 1e-6f), gam, bet};  // blas.zig:141-143
 }
 
 // x_norm = (input - m) * inv (blas.zig:137-146); output = act(x_norm * scale
@@ -700,41 +592,6 @@ __global__ __launch_bounds__(BS) void bn_fwd_coop_kernel(const float *input, flo
 
 // ---- backward -----------------------------------------------------------------
 
-// Per channel: s0 = sum(d1), s1 = sum(d1 * x_norm), s2 = sum(d2),
-// s3 = sum(d2 * (x - m)), where d1 = delta * gradient(y) (activations.zig:
-// 127-143) and d2 = d1 * scale (the scale_bias on delta, batchnorm.zig:165).
-struct BwdFin {
-    const float *variance;
-    float *bias_updates, *scale_updates, *mean_delta, *variance_delta;
-    __device__ void values(uint32_t f, const Sums<4> &r, float &md, float &vd) const {
-        const float v = variance[f];
-        md = (float)r.s[2] * (-1.0f / sqrtf(v + 1e-5f));            // blas.zig:155
-        vd = ((float)r.s[3] * -0.5f) * pow_m1p5(v + 1e-5f);          // blas.zig:176
-    }
-    // met == false (a one-launch pass whose channel barrier gave up):
-    // mean_delta and variance_delta are written (NaN), but nothing is added
-    // to the updates, which accumulate across calls.
-    __device__ void write(uint32_t f, const Sums<4> &r, float md, float vd, bool met = true) const {
-        if (met) {
-            bias_updates[f] = bias_updates[f] + (float)r.s[0];   // blas.zig:79
-            scale_updates[f] = scale_updates[f] + (float)r.s[1]; // blas.zig:98
-        }
-        mean_delta[f] = md;
-        variance_delta[f] = vd;
-    }
-    __device__ void operator()(uint32_t f, const Sums<4> &r) const {
-        float md, vd;
-        values(f, r, md, vd);
-        write(f, r, md, vd);
-    }
-};
-
-template <int A>
-__device__ __forceinline__ float grad_delta(float d, float y) {
-    if constexpr (A == kLinear) return d;  // activations.zig:129: linear leaves delta alone
-    else return d * gradient<A>(y);
-}
-
 template <int A>
 __device__ __forceinline__ void acc_bwd(float4 y, float4 d, float4 xn, float4 x, float m, float gam,
                                         double (&a)[4]) {
@@ -797,22 +654,6 @@ __global__ __launch_bounds__(BS) void bn_bwd_sums_kernel(const float *y, const f
     }
 }
 
-struct BwdParams {
-    const float *mean, *variance, *mean_delta, *variance_delta, *scales;
-    float denom;  // f32(spatial * batch), blas.zig:191
-};
-
-// What the backward apply pass needs of channel f.
-struct BwdChan {
-    float m, inv, vd2, mdn, gam;
-};
-
-__device__ __forceinline__ BwdChan bwd_chan(const BwdParams &p, uint32_t f, float md, float vd) {
-    return {p.mean[f], 1.0f / sqrtf(p.variance[f] + 1e-5f), vd * 2.0f, md / p.denom, p.scales[f]};
-}
-
-// delta = d2 * inv + ((vd * 2) * (x - m)) / N + md / N (blas.zig:180-204) on
-// d2 = delta * gradient(y) * scale.
 template <int A>
 __device__ __forceinline__ float4 bwd_elem(float4 y, float4 d, float4 x, const BwdChan &c, float denom) {
     float4 o;
@@ -1308,26 +1149,6 @@ bool no_spills() {
     return v == 1;
 }
 
-struct Shape {
-    uint32_t B, F, S, n;
-};
-
-struct FwdArgs {
-    Shape sh;
-    bool train;
-    const float *input;
-    float *output, *x, *x_norm, *mean, *variance, *rolling_mean, *rolling_variance;
-    const float *scales, *biases;
-};
-
-struct BwdArgs {
-    Shape sh;
-    const float *y;
-    float *delta;
-    const float *x, *x_norm, *mean, *variance, *scales;
-    float *bias_updates, *scale_updates, *mean_delta, *variance_delta;
-};
-
 // Split of a reduction pass over the channels of a shape.
 template <int NS>
 RedGeom sums_geom(const Shape &sh, uint32_t streams) {
@@ -1619,12 +1440,12 @@ int dkz_batchnorm_forward(int batch, int filters, int spatial, int activation, i
     const int n = (int)n64;
     const bool fast = n64 > 0 && spatial % 4 == 0 && aligned16(input) && aligned16(output) && aligned16(x) &&
                       (!train || aligned16(x_norm));
-    if (fast) {
-        const FwdArgs a{{(uint32_t)batch, (uint32_t)filters, (uint32_t)spatial, (uint32_t)n},
-                        train != 0, input, output, x, x_norm, mean, variance, rolling_mean, rolling_variance,
-                        scales, biases};
-        return Tables::fwd[activation](a);
-    }
+    const FwdArgs a{{(uint32_t)batch, (uint32_t)filters, (uint32_t)spatial, (uint32_t)n},
+                    train != 0, input, output, x, x_norm, mean, variance, rolling_mean, rolling_variance,
+                    scales, biases};
+    if (fast) return Tables::fwd[activation](a);
+    int rc = 0;
+    if (n64 > 0 && bn_forward_ragged(activation, a, &rc)) return rc;
     // The per-op sequence of batchnorm.zig:129-153 and convolutional.zig:269.
     if (input != output) DKZ_TRY(dkz_copy(n, input, output));
     DKZ_TRY(dkz_copy(n, output, x));
@@ -1659,12 +1480,12 @@ int dkz_batchnorm_backward(int batch, int filters, int spatial, int activation, 
     const int n = (int)n64;
     const bool fast = n64 > 0 && spatial % 4 == 0 && aligned16(delta) && aligned16(x) && aligned16(x_norm) &&
                       (activation == kLinear || aligned16(output));
-    if (fast) {
-        const BwdArgs a{{(uint32_t)batch, (uint32_t)filters, (uint32_t)spatial, (uint32_t)n},
-                        output, delta, x, x_norm, mean, variance, scales,
-                        bias_updates, scale_updates, mean_delta, variance_delta};
-        return Tables::bwd[activation](a);
-    }
+    const BwdArgs a{{(uint32_t)batch, (uint32_t)filters, (uint32_t)spatial, (uint32_t)n},
+                    output, delta, x, x_norm, mean, variance, scales,
+                    bias_updates, scale_updates, mean_delta, variance_delta};
+    if (fast) return Tables::bwd[activation](a);
+    int rc = 0;
+    if (n64 > 0 && bn_backward_ragged(activation, a, &rc)) return rc;
     // convolutional.zig:280 and the per-op sequence of batchnorm.zig:155-174.
     DKZ_TRY(dkz_gradient_array(output, n, activation, delta));
     DKZ_TRY(dkz_backward_bias(bias_updates, delta, batch, filters, spatial));
