@@ -37,31 +37,57 @@ constexpr uint32_t kCus = 256;
 // 1450 of them (4 x 362), 128x64 and 64x128 900 (2 x 450), 64x64 520; alone 1900,
 // 1300 and 900. Smaller tiles fill the chip at the price of more LDS traffic
 // and splitting per product.
+//
+// stream != 0: tiles that fill no whole round of the chip (`occupancy`
+// workgroups a CU) have their slabs laid end to end and cut into equal runs of
+// `stream` slabs, one a workgroup, so that the round ends everywhere at once.
+// Where a uniform split leaves CUs with one workgroup more than others, or the
+// last round nearly empty, that costs more than the pieces' traffic:
+// [64,128,56,56]->128 3x3 (1568 tiles, 3.06 rounds) and [32,512,13,13]->1024
+// (172 and 288 tiles).
 struct Tiling {
-    uint32_t bm, bn, splits, k_chunk;
+    uint32_t bm, bn, splits, k_chunk, full_tiles, stream;
 };
-Tiling pick_tiling(uint64_t m, uint64_t n, uint64_t k, uint64_t z, uint64_t max_splits) {
+Tiling pick_tiling(uint64_t m, uint64_t n, uint64_t k, uint64_t z, uint64_t max_splits, uint64_t partial_floats) {
     struct Cost {
-        uint32_t bm, bn;
+        uint32_t bm, bn, occupancy;
         double full, alone;
+        // Of `slabs` slabs in each of per_cu workgroups.
+        double cycles(uint64_t slabs, uint64_t per_cu) const {
+            const uint64_t rest = per_cu % occupancy;
+            return (double)slabs * ((double)(per_cu - rest) * full + (rest ? std::max(alone, (double)rest * full) : 0.0));
+        }
     };
-    static constexpr Cost kTiles[] = {{128, 128, 1450, 1900}, {128, 64, 900, 1300}, {64, 128, 900, 1300}, {64, 64, 520, 900}, {32, 128, 520, 900}};
+    static constexpr Cost kTiles[] = {
+        {128, 128, 2, 1450, 1900}, {128, 64, 3, 900, 1300}, {64, 128, 3, 900, 1300}, {64, 64, 4, 520, 900}, {32, 128, 4, 520, 900}};
     static constexpr uint8_t kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 56, 64, 80, 96, 112, 128, 160, 192, 224, 255};
-    const uint32_t slabs = div_up(k, kBK);
-    Tiling best{64, 64, 1, slabs * kBK};
+    constexpr double kFloats = 2.0 * 4 / 2000;  // cycles a float of partials: ~4.2 TB/s at 2.1 GHz
+    const uint64_t slabs = div_up(k, kBK);
+    Tiling best{64, 64, 1, (uint32_t)slabs * kBK, 0, 0};
     double least = 1e300;
     for (const Cost &t : kTiles) {
         const uint64_t tiles = (uint64_t)div_up(m, t.bm) * div_up(n, t.bn) * z;
         for (const uint32_t want : kSplits) {
-            const uint32_t chunk = (slabs + want - 1) / want, splits = chunk ? (slabs + chunk - 1) / chunk : 1;
+            const uint64_t chunk = (slabs + want - 1) / want, splits = chunk ? (slabs + chunk - 1) / chunk : 1;
             if (want > 1 && (want > max_splits || chunk < 4 || tiles * splits > 4 * kCus + tiles)) break;
-            const double per_cu = (double)((tiles * splits + kCus - 1) / kCus);
-            double cycles = 3000 + (double)chunk * std::max(t.alone, per_cu * t.full);
-            if (splits > 1) cycles += 6000 + 2.0 * 4 * m * n * splits / 2000;  // ~4.2 TB/s at 2.1 GHz
+            double cycles = 3000 + t.cycles(chunk, (tiles * splits + kCus - 1) / kCus);
+            if (splits > 1) cycles += 6000 + kFloats * m * n * splits;
             if (cycles < least) {
                 least = cycles;
-                best = {t.bm, t.bn, splits, chunk * kBK};
+                best = {t.bm, t.bn, (uint32_t)splits, (uint32_t)chunk * kBK, 0, 0};
             }
+        }
+        // Runs of at least four slabs, at most 34 pieces a tile.
+        const uint64_t slots = kCus * t.occupancy, rest = tiles % slots, line = rest * slabs;
+        const uint64_t run = std::max<uint64_t>({(line + slots - 1) / slots, (slabs + 31) / 32, 4});
+        if (max_splits == 0 || rest == 0 || run >= slabs || line + run >= 1ull << 31) continue;
+        const uint64_t runs = (line + run - 1) / run, floats = (runs + rest) * t.bm * t.bn;
+        if (floats > partial_floats) continue;
+        const double cycles = 3000 + t.cycles(slabs, (tiles - rest) / kCus) + t.cycles(run, (runs + kCus - 1) / kCus) + 6000 +
+                              2000.0 * (double)((slabs / run + 9) / 8) + kFloats * floats;
+        if (cycles < least) {
+            least = cycles;
+            best = {t.bm, t.bn, 1, (uint32_t)slabs * kBK, (uint32_t)(tiles - rest), (uint32_t)run};
         }
     }
     return best;
@@ -70,20 +96,32 @@ Tiling pick_tiling(uint64_t m, uint64_t n, uint64_t k, uint64_t z, uint64_t max_
 // Runs a product of g's operands over `z` grid rows (one when K may be split).
 template <Operand AK, Operand BK>
 int launch_split(const char *name, SplitArgs g, uint32_t z) {
-    uint64_t max_splits = 1;
+    uint64_t max_splits = 0, left = 0;
     Scratch sc{};
     if (z == 1 && g.phases == 0 && g.partial != nullptr && g.k >= 8 * kBK) {
         DKZ_TRY(device_scratch(&sc));
-        const uint64_t left = (uint64_t)(sc.gemm + sc.gemm_floats - g.partial) / ((uint64_t)g.m * g.n);
-        max_splits = std::max<uint64_t>(1, std::min<uint64_t>(255, left));
+        left = (uint64_t)(sc.gemm + sc.gemm_floats - g.partial);
+        max_splits = std::max<uint64_t>(1, std::min<uint64_t>(255, left / ((uint64_t)g.m * g.n)));
     }
     constexpr bool kWide = BK == kGatherWide || BK == kTapWide;
-    const Tiling t = kWide ? Tiling{64, 64, 1, div_up(g.k, kBK) * kBK} : pick_tiling(g.m, g.n, g.k, z, max_splits);
+    const Tiling t = kWide ? Tiling{64, 64, 1, div_up(g.k, kBK) * kBK, 0, 0}
+                           : pick_tiling(g.m, g.n, g.k, z, max_splits, left);
     g.tiles_m = div_up(g.m, t.bm);
     g.tiles_n = div_up(g.n, t.bn);
     g.splits = t.splits;
     g.k_chunk = t.k_chunk;
-    const uint64_t total = (uint64_t)g.tiles_m * g.tiles_n * g.splits;
+    uint64_t total = (uint64_t)g.tiles_m * g.tiles_n * g.splits;
+    const uint32_t streamed = t.stream ? (uint32_t)(total - t.full_tiles) : 0;
+    if (t.stream) {
+        const uint32_t slabs = div_up(g.k, kBK);
+        g.full_tiles = t.full_tiles;
+        g.stream_len = t.stream;
+        g.stream_slabs = streamed * slabs;
+        g.div_tile_slabs = make_fastdiv(slabs);
+        g.tile_bm = t.bm;
+        g.tile_bn_log2 = t.bn == 128 ? 7 : 6;
+        total = t.full_tiles + div_up(g.stream_slabs, t.stream);
+    }
     DKZ_REQUIRE(total <= 0x7fffffffull);
     const dim3 grid((uint32_t)total, z), block(kBlock);
     if constexpr (kWide) {
@@ -95,9 +133,14 @@ int launch_split(const char *name, SplitArgs g, uint32_t z) {
         else if (t.bm == 32) DKZ_TRY(launch(name, gemm_split_kernel<32, 128, AK, BK>, grid, block, g));
         else DKZ_TRY(launch(name, gemm_split_kernel<64, 64, AK, BK>, grid, block, g));
     }
+    const bool v4 = g.n % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.c) && g.npos % 4 == 0 && g.c_img % 4 == 0;
+    if (t.stream) {
+        const dim3 blocks(streamed * (t.bm * t.bn / 4 / kBlock));
+        return v4 ? launch(name, stream_reduce_kernel<true>, blocks, block, g)
+                  : launch(name, stream_reduce_kernel<false>, blocks, block, g);
+    }
     if (g.splits == 1) return 0;
     const uint64_t mn = (uint64_t)g.m * g.n;
-    const bool v4 = g.n % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.c) && g.npos % 4 == 0 && g.c_img % 4 == 0;
     // Eight partials in flight; 32 where a small C has so many that their round
     // trips would add up.
     const bool many = g.splits > 32;

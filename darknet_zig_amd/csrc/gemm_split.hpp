@@ -96,6 +96,11 @@ struct SplitArgs {
     uint32_t m, n, k, lda, ldb, ldc;
     float alpha, beta;
     uint32_t tiles_m, tiles_n, splits, k_chunk;
+    // stream_len != 0 (splits 1, one grid row): tiles from full_tiles on are
+    // streamed, stream_len slabs of the line (tile, slab) a workgroup.
+    uint32_t full_tiles, stream_len, stream_slabs;  // stream_slabs: the whole line's
+    FastDiv div_tile_slabs;
+    uint32_t tile_bm, tile_bn_log2;
     // Batched launches (z = blockIdx.y): A at a + (z % zgroups) * a_z, B at
     // b + z * b_z, C at c + z * c_z.
     uint32_t zgroups;
@@ -130,13 +135,13 @@ __device__ __forceinline__ float *c_column(float *c, uint32_t j, const SplitArgs
     return c + (size_t)(g.ph_s * yq + py) * g.ph_w + g.ph_s * xq + px;
 }
 
-__device__ __forceinline__ void tile_of(uint32_t w, const SplitArgs &g, uint32_t &tm, uint32_t &tn, uint32_t &split) {
-    const uint32_t tiles = g.tiles_m * g.tiles_n;
-    const uint32_t total = tiles * g.splits;
-    uint32_t t = w;
-    if (total % kXcds == 0) t = (w % kXcds) * (total / kXcds) + w / kXcds;
-    split = t / tiles;
-    t -= split * tiles;
+// Consecutive workgroups go round the XCDs: gives each XCD a run of neighbours.
+__device__ __forceinline__ uint32_t xcd_order(uint32_t w, uint32_t total) {
+    return total % kXcds == 0 ? (w % kXcds) * (total / kXcds) + w / kXcds : w;
+}
+
+// Tile t's row and column of tiles: groups of kGroupM rows, column by column.
+__device__ __forceinline__ void tile_at(uint32_t t, const SplitArgs &g, uint32_t &tm, uint32_t &tn) {
     const uint32_t per_group = kGroupM * g.tiles_n;
     const uint32_t first_m = (t / per_group) * kGroupM;
     const uint32_t gsize = g.tiles_m - first_m < (uint32_t)kGroupM ? g.tiles_m - first_m : (uint32_t)kGroupM;
@@ -636,17 +641,43 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
         k_chunk = lda = k_all;
         a_z = (uint64_t)g.m * k_all;
     }
-    uint32_t tm, tn, split;
-    tile_of(blockIdx.x, g, tm, tn, split);
     const float *ga = a_base + (size_t)(z % g.zgroups) * a_z;
     const float *gb = g.b + (size_t)z * g.b_z;
     float *gc = g.c + (size_t)z * g.c_z;
-    const uint32_t m0 = tm * BM, n0 = tn * BN;
-    const uint32_t kbeg = split * k_chunk;
-    const uint32_t kend = kbeg + k_chunk < k_all ? kbeg + k_chunk : k_all;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm0 = BM == 32 ? 0 : (wave >> 1) * WM, wn0 = (BM == 32 ? wave : wave & 1) * WN;
     const int half = lane >> 5, l32 = lane & 31;
+
+    // One K range of one tile; or a run of the streamed line: the last slabs of
+    // a tile, the first ones of the next. Piece (workgroup b, tile t) has
+    // partial tile b + t (along the line at least one of the two advances).
+    const bool streams = g.stream_len != 0 && blockIdx.x >= g.full_tiles;
+    uint32_t block = blockIdx.x, line = 0, line_end = 0;
+    if (streams) {
+        block = xcd_order(block - g.full_tiles, gridDim.x - g.full_tiles);
+        line = block * g.stream_len;
+        line_end = min(line + g.stream_len, g.stream_slabs);
+    }
+#pragma unroll 1
+    do {
+    uint32_t tm, tn, kbeg, kend, slot = 0;
+    if (streams) {
+        const uint32_t t = fdiv(line, g.div_tile_slabs), first = line - t * g.div_tile_slabs.d;
+        const uint32_t len = min(g.div_tile_slabs.d - first, line_end - line);
+        tile_at(g.full_tiles + t, g, tm, tn);
+        kbeg = first * kBK;
+        kend = min(kbeg + len * kBK, k_all);
+        slot = block + t;
+        line += len;
+    } else {
+        const uint32_t tiles = g.stream_len != 0 ? g.full_tiles : g.tiles_m * g.tiles_n;
+        uint32_t t = xcd_order(block, tiles * g.splits);
+        slot = t / tiles;
+        tile_at(t - slot * tiles, g, tm, tn);
+        kbeg = slot * k_chunk;
+        kend = kbeg + k_chunk < k_all ? kbeg + k_chunk : k_all;
+    }
+    const uint32_t m0 = tm * BM, n0 = tn * BN;
 
     // Two register sets: slab s is loaded into set s & 1.
     typename Loader<AK, RA>::type sa[2];
@@ -820,10 +851,14 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
         for (int ti = 0; ti < TM; ++ti) {
             const uint32_t i0 = m0 + wm0 + ti * 32 + half * 4;
             const auto row = [&](int r) { return i0 + (r >> 2) * 8 + (r & 3); };
-            float *to = g.splits > 1 ? g.partial + (size_t)split * g.m * g.n + j : ccol;
-            const uint32_t ld = g.splits > 1 ? g.n : g.ldc;
+            // A K range's partial is a whole m x n one, a streamed piece's its tile.
+            const bool part = streams || g.splits > 1;
+            float *to = !part     ? ccol
+                        : streams ? g.partial + (size_t)slot * (BM * BN) + (j - n0) - (size_t)m0 * BN
+                                  : g.partial + (size_t)slot * g.m * g.n + j;
+            const uint32_t ld = !part ? g.ldc : streams ? BN : g.n;
             float out[16];
-            if (g.splits > 1) {
+            if (part) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) out[r] = big[ti][tj][r];
             } else if (g.beta == 0.0f) {
@@ -846,6 +881,7 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
             }
         }
     }
+    } while (line < line_end);
 }
 
 // The split-K epilogue: adds a tile's partials in split order, then as the
@@ -876,6 +912,50 @@ __global__ __launch_bounds__(kBlock) void split_reduce_kernel(SplitArgs g) {
 #pragma unroll
     for (uint32_t x = 0; x < kW; ++x) reinterpret_cast<float *>(&o)[x] = gemm_out(cp + x, s[x], g.alpha, g.beta);
     *reinterpret_cast<T *>(cp) = o;
+}
+
+// The streamed tiles' epilogue: adds a tile's pieces in k order, then as above.
+// A lane takes four consecutive columns of one row, eight pieces in flight; V4:
+// they are 16 aligned bytes of C.
+template <bool V4>
+__global__ __launch_bounds__(kBlock) void stream_reduce_kernel(SplitArgs g) {
+    constexpr int kPieces = 8;
+    const uint32_t tile_floats = g.tile_bm << g.tile_bn_log2;
+    const uint32_t e = 4 * (blockIdx.x * kBlock + threadIdx.x), t = e / tile_floats, at = e - t * tile_floats;
+    uint32_t tm, tn;
+    tile_at(g.full_tiles + t, g, tm, tn);
+    const uint32_t i = tm * g.tile_bm + (at >> g.tile_bn_log2);
+    const uint32_t j = (tn << g.tile_bn_log2) + (at & ((1u << g.tile_bn_log2) - 1));
+    if (i >= g.m || j >= g.n) return;
+    const uint32_t slabs = g.div_tile_slabs.d;
+    const uint32_t first = t * slabs / g.stream_len, last = ((t + 1) * slabs - 1) / g.stream_len;
+    const float *from = g.partial + at + (size_t)t * tile_floats;
+    float s[4] = {};
+    for (uint32_t b = first; b <= last; b += kPieces) {
+        float4 p[kPieces];
+#pragma unroll
+        for (int u = 0; u < kPieces; ++u)
+            p[u] = b + u <= last ? *reinterpret_cast<const float4 *>(from + (size_t)(b + u) * tile_floats)
+                                 : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+        for (int u = 0; u < kPieces; ++u)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) s[x] += ::dkz::lane(p[u], x);
+    }
+    if constexpr (V4) {
+        float *cp = c_column(g.c, j, g, 0, 0) + (size_t)i * g.ldc;
+        float4 o;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) ::dkz::lane(o, x) = gemm_out(cp + x, s[x], g.alpha, g.beta);
+        *reinterpret_cast<float4 *>(cp) = o;
+    } else {
+#pragma unroll
+        for (uint32_t x = 0; x < 4; ++x) {
+            if (j + x >= g.n) break;
+            float *cp = c_column(g.c, j + x, g, 0, 0) + (size_t)i * g.ldc;
+            *cp = gemm_out(cp, s[x], g.alpha, g.beta);
+        }
+    }
 }
 
 }  // namespace
