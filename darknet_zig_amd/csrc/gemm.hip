@@ -9,7 +9,8 @@
 // the tile grid, each summing one range of K into a partial tile in the
 // library's scratch, and a second kernel adds a tile's partials in split order
 // and applies alpha and beta -- deterministic, no atomics. The epilogue follows
-// gemm.zig:121-131 then :180-184: beta == 0 clears C (NaN included), beta == 1
+// gemm.zig:121-131 then :180-184 (so do the streamed tiles' pieces, see
+// pick_tiling): beta == 0 clears C (NaN included), beta == 1
 // keeps it, anything else scales it; then C += alpha*acc.
 //
 // Workgroups take tiles in groups of 8 tile-rows, so that the tiles running
@@ -41,10 +42,13 @@ constexpr uint32_t kCus = 256;
 // stream != 0: tiles that fill no whole round of the chip (`occupancy`
 // workgroups a CU) have their slabs laid end to end and cut into equal runs of
 // `stream` slabs, one a workgroup, so that the round ends everywhere at once.
-// Where a uniform split leaves CUs with one workgroup more than others, or the
-// last round nearly empty, that costs more than the pieces' traffic:
-// [64,128,56,56]->128 3x3 (1568 tiles, 3.06 rounds) and [32,512,13,13]->1024
-// (172 and 288 tiles).
+// Where whole tiles or uniform ranges leave some CUs with a workgroup more than
+// others, or the last round nearly empty, that costs more than the pieces'
+// traffic and the second launch: [64,128,56,56]->128 3x3 (1568 tiles, 3.06
+// rounds) 435 us in whole tiles, 402 streamed; [32,512,13,13]->1024 (172 and 288
+// tiles) both gradients 851 us in uniform ranges, 729 streamed. Below one round,
+// where a uniform range a workgroup fits (2048^3 in two, [256,4096]x[4096,1000]
+// in eight), the two cost the same and the uniform one is taken.
 struct Tiling {
     uint32_t bm, bn, splits, k_chunk, full_tiles, stream;
 };
