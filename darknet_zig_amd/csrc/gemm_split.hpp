@@ -416,8 +416,10 @@ struct GatherWideLoad : ColBase<R> {
 
 // The quad of k at k0 + 4 * (tid % 4) of a weight gradient: its image (from the
 // split's first one on) and first position; `in` says whether it is there. The
-// host gives the kernels that use it images, positions and image sides below
-// 2^24, so that all products but those with the image stride are 24-bit ones.
+// host gives the narrow loaders images, positions and image sides below 2^24, so
+// that all their products but those with the image stride are 24-bit ones; WIDE
+// takes any.
+template <bool WIDE>
 struct Quad {
     uint32_t img, p;
     bool in;
@@ -426,7 +428,7 @@ struct Quad {
         const uint32_t i = fdiv_select(k, g.div_kpos4);
         in = k < kend;
         img = i - img0;
-        p = k - __umul24(i, g.div_kpos4.d);
+        p = k - (WIDE ? i * g.div_kpos4.d : __umul24(i, g.div_kpos4.d));
     }
 };
 
@@ -461,7 +463,7 @@ struct SegLoad : QuadBase<R> {
                                                 0x80000000u, 0x00020000);
     }
     __device__ __forceinline__ void load(uint32_t k0, uint32_t kend, int tid, uint64_t img_stride, const SplitArgs &g) {
-        const Quad q(k0, kend, img0, tid, g);
+        const Quad<false> q(k0, kend, img0, tid, g);
         const uint32_t p = ODD ? min(q.p, g.kpos - 4) : q.p, d = q.p - p;
         const uint32_t off = 4 * (q.img * (uint32_t)img_stride + p);
 #pragma unroll
@@ -502,7 +504,7 @@ struct TapLoad : QuadBase<R> {
         buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + (size_t)img0 * g.b_img), 0, 0x80000000u, 0x00020000);
     }
     __device__ __forceinline__ void load(uint32_t k0, uint32_t kend, int tid, const ConvGeom &cv, const SplitArgs &g) {
-        const Quad q(k0, kend, img0, tid, g);
+        const Quad<false> q(k0, kend, img0, tid, g);
         const uint32_t h = fdiv_select(q.p, cv.div_wo), last = __umul24(cv.div_wo.d - 1, cv.stride);
         uint32_t y = __umul24(h, cv.stride), x = __umul24(q.p - __umul24(h, cv.div_wo.d), cv.stride);
         uint32_t pos = q.img * (uint32_t)g.b_img + __umul24(y, cv.W) + x;
@@ -532,7 +534,7 @@ struct QuadWideLoad : QuadBase<R> {
     using QuadBase<R>::row;
     __device__ __forceinline__ void load(const float *base, uint32_t r0, uint32_t rows, uint32_t k0, uint32_t kend, int tid,
                                          uint64_t img_stride, const ConvGeom &cv, const SplitArgs &g) {
-        const Quad q(k0, kend, 0, tid, g);
+        const Quad<true> q(k0, kend, 0, tid, g);
 #pragma unroll
         for (int l = 0; l < kL; ++l) {
             const uint32_t f = tid + l * kBlock, r = r0 + (f / 4 < rows ? f / 4 : rows - 1);
