@@ -52,7 +52,12 @@ constexpr uint32_t kCus = 256;
 struct Tiling {
     uint32_t bm, bn, splits, k_chunk, full_tiles, stream;
 };
-Tiling pick_tiling(uint64_t m, uint64_t n, uint64_t k, uint64_t z, uint64_t max_splits, uint64_t partial_floats) {
+// K ranges go to 1024 of them: weight gradients over large maps have K in the
+// millions and a tile or two ([2,3,2048,2048]->16 3x3: 525 thousand slabs, one tile).
+//
+// wide: the kernels with 64-bit addresses, built for 64x64 tiles alone.
+constexpr uint64_t kMaxSplits = 1024;
+Tiling pick_tiling(uint64_t m, uint64_t n, uint64_t k, uint64_t z, uint64_t max_splits, uint64_t partial_floats, bool wide) {
     struct Cost {
         uint32_t bm, bn, occupancy;
         double full, alone;
@@ -64,12 +69,14 @@ Tiling pick_tiling(uint64_t m, uint64_t n, uint64_t k, uint64_t z, uint64_t max_
     };
     static constexpr Cost kTiles[] = {
         {128, 128, 2, 1450, 1900}, {128, 64, 3, 900, 1300}, {64, 128, 3, 900, 1300}, {64, 64, 4, 520, 900}, {32, 128, 4, 520, 900}};
-    static constexpr uint8_t kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 56, 64, 80, 96, 112, 128, 160, 192, 224, 255};
+    static constexpr uint16_t kSplits[] = {1,  2,  3,  4,  5,  6,   7,   8,   10,  12,  14,  16,  20,  24,  28,  32,        40,
+                                           48, 56, 64, 80, 96, 112, 128, 160, 192, 224, 256, 320, 384, 512, 640, 768, kMaxSplits};
     constexpr double kFloats = 2.0 * 4 / 2000;  // cycles a float of partials: ~4.2 TB/s at 2.1 GHz
     const uint64_t slabs = div_up(k, kBK);
     Tiling best{64, 64, 1, (uint32_t)slabs * kBK, 0, 0};
     double least = 1e300;
     for (const Cost &t : kTiles) {
+        if (wide && (t.bm != 64 || t.bn != 64)) continue;
         const uint64_t tiles = (uint64_t)div_up(m, t.bm) * div_up(n, t.bn) * z;
         for (const uint32_t want : kSplits) {
             const uint64_t chunk = (slabs + want - 1) / want, splits = chunk ? (slabs + chunk - 1) / chunk : 1;
@@ -105,11 +112,10 @@ int launch_split(const char *name, SplitArgs g, uint32_t z) {
     if (z == 1 && g.phases == 0 && g.partial != nullptr && g.k >= 8 * kBK) {
         DKZ_TRY(device_scratch(&sc));
         left = (uint64_t)(sc.gemm + sc.gemm_floats - g.partial);
-        max_splits = std::max<uint64_t>(1, std::min<uint64_t>(255, left / ((uint64_t)g.m * g.n)));
+        max_splits = std::max<uint64_t>(1, std::min<uint64_t>(kMaxSplits, left / ((uint64_t)g.m * g.n)));
     }
     constexpr bool kWide = BK == kGatherWide || BK == kTapWide;
-    const Tiling t = kWide ? Tiling{64, 64, 1, div_up(g.k, kBK) * kBK, 0, 0}
-                           : pick_tiling(g.m, g.n, g.k, z, max_splits, left);
+    const Tiling t = pick_tiling(g.m, g.n, g.k, z, max_splits, left, kWide);
     g.tiles_m = div_up(g.m, t.bm);
     g.tiles_n = div_up(g.n, t.bn);
     g.splits = t.splits;
@@ -129,7 +135,7 @@ int launch_split(const char *name, SplitArgs g, uint32_t z) {
     DKZ_REQUIRE(total <= 0x7fffffffull);
     const dim3 grid((uint32_t)total, z), block(kBlock);
     if constexpr (kWide) {
-        return launch(name, gemm_split_kernel<64, 64, AK, BK>, grid, block, g);
+        DKZ_TRY(launch(name, gemm_split_kernel<64, 64, AK, BK>, grid, block, g));
     } else {
         if (t.bm == 128 && t.bn == 128) DKZ_TRY(launch(name, gemm_split_kernel<128, 128, AK, BK>, grid, block, g));
         else if (t.bm == 128) DKZ_TRY(launch(name, gemm_split_kernel<128, 64, AK, BK>, grid, block, g));
@@ -529,9 +535,6 @@ int dkz_convolution_weight_gradient(int batch, int groups, int channels, int hei
     DKZ_REQUIRE(ksize != 1 || npos <= (uint64_t)height * width);  // the input is read as a k x n matrix
     Scratch sc;
     DKZ_TRY(device_scratch(&sc));
-    // k = image * npos4 + position, each image's positions rounded up to a
-    // multiple of four.
-    const uint64_t npos4 = (npos + 3) / 4 * 4;
     SplitArgs g{};
     g.m = (uint32_t)m;
     g.n = (uint32_t)kw;
@@ -540,35 +543,53 @@ int dkz_convolution_weight_gradient(int batch, int groups, int channels, int hei
     g.beta = 1.0f;
     g.partial = sc.gemm;
     g.zgroups = 1;
-    g.kpos = (uint32_t)npos;
-    g.div_kpos4 = make_fastdiv((uint32_t)npos4);
+    g.krow = (uint32_t)npos;
     g.a_img = (uint64_t)groups * m * npos;
     g.b_img = (uint64_t)groups * in_group;
-    // ksize 1 reads the input as a k x n matrix: rows of npos positions.
-    g.cv = ksize == 1 ? conv_geom(1, npos, npos, 1, 1, 1, 0, 0)
-                      : conv_geom((uint64_t)height, (uint64_t)width, wo, (uint32_t)ksize, (uint32_t)ksize, (uint32_t)stride, pad, pad);
-    // The 32-bit loaders: a split's images and one row tile within 2^31 bytes,
-    // 24-bit products, at least one whole quad an image.
-    constexpr uint64_t k24 = 1u << 24;
-    const bool narrow = npos >= 4 && npos4 < k24 && (uint64_t)batch < k24 && (uint64_t)height < k24 && (uint64_t)width < k24 &&
-                        (uint64_t)stride < k24 && ((uint64_t)batch * g.a_img + 128 * npos) * 4 < kMaxOffset &&
-                        ((uint64_t)batch * g.b_img + std::max<uint64_t>(128 * npos, ((uint64_t)height + 2 * (uint64_t)pad) * width)) * 4 < kMaxOffset;
+    // The narrow loaders: an image within 2^31 bytes, at least one whole quad
+    // an image, and 24-bit products: a map of 2^24 positions or more goes
+    // through them in bands of output rows (of positions, where ksize 1 reads
+    // the input as a k x n matrix). The others take 64-bit addresses element by
+    // element: half the speed or less.
+    constexpr uint64_t k24 = 1u << 24, kBand = k24 - 4;
+    const uint64_t img_bytes = 4 * std::max(g.a_img, g.b_img), row = ksize == 1 ? 4 : wo;
+    const bool narrow = npos >= 4 && row <= kBand && img_bytes < kMaxOffset &&
+                        (ksize == 1 || ((uint64_t)height < k24 && (uint64_t)width < k24 && (uint64_t)stride < k24));
+    const uint64_t rows = div_up(npos, row), bands = narrow && npos > kBand ? div_up(rows, kBand / row) : 1;
+    const uint64_t band = std::min(npos, div_up(rows, bands) * row);
+    // k = image * band4 + position, each band's positions rounded up to a
+    // multiple of four. As many images a product as keep k below 2^31 and, for
+    // the narrow loaders, the images below 2^24 and within 2^31 bytes; later
+    // ones add to the same updates. [64,3,416,416]->64 3x3 (2.8 GB of delta) in
+    // two products 1.2 ms, where one through the 64-bit loaders took 820 ms.
+    // (band4 may be 2^31, of a single image.)
+    const auto up4 = [](uint64_t x) { return (x + 3) / 4 * 4; };
+    uint64_t most = std::min<uint64_t>((uint64_t)batch, std::max<uint64_t>(kMaxElems / up4(band), 1));
+    if (narrow) most = std::min({most, k24 - 1, (kMaxOffset - 1) / img_bytes});
+    if (bands > 1) most = 1;
     constexpr const char *kName = "convolution_weight_gradient";
-    // As many images a product as keep k below 2^31 (all of them but where
-    // images have one or two positions); later ones add to the same updates.
-    const uint64_t most = std::min<uint64_t>((uint64_t)batch, kMaxElems / npos4);
     for (int j = 0; j < groups; ++j) {
         for (uint64_t i0 = 0; i0 < (uint64_t)batch; i0 += most) {
-            SplitArgs gj = g;
-            gj.k = (uint32_t)(std::min<uint64_t>(most, (uint64_t)batch - i0) * npos4);
-            gj.a = delta + i0 * g.a_img + (uint64_t)j * m * npos;
-            gj.b = input + i0 * g.b_img + (uint64_t)j * in_group;
-            gj.c = weight_updates + (uint64_t)j * m * kw;
-            if (!narrow) DKZ_TRY((launch_split<kSegWide, kTapWide>(kName, gj, 1)));
-            else if (ksize == 1 && npos % 4 == 0) DKZ_TRY((launch_split<kSeg, kSeg>(kName, gj, 1)));
-            else if (ksize == 1) DKZ_TRY((launch_split<kSegOdd, kSegOdd>(kName, gj, 1)));
-            else if (npos % 4 == 0) DKZ_TRY((launch_split<kSeg, kTap>(kName, gj, 1)));
-            else DKZ_TRY((launch_split<kSegOdd, kTap>(kName, gj, 1)));
+            for (uint64_t p0 = 0; p0 < npos; p0 += band) {
+                SplitArgs gj = g;
+                const uint64_t kpos = std::min(band, npos - p0), kpos4 = up4(kpos);
+                gj.kpos = (uint32_t)kpos;
+                gj.div_kpos4 = make_fastdiv((uint32_t)kpos4);
+                gj.k = (uint32_t)(std::min<uint64_t>(most, (uint64_t)batch - i0) * kpos4);
+                gj.a = delta + i0 * g.a_img + (uint64_t)j * m * npos + p0;
+                gj.b = input + i0 * g.b_img + (uint64_t)j * in_group + (ksize == 1 ? p0 : 0);
+                gj.c = weight_updates + (uint64_t)j * m * kw;
+                // A band starts p0 / wo output rows down (modulo 2^32, as the
+                // loaders' bounds tests are).
+                gj.cv = ksize == 1 ? conv_geom(1, npos, npos, 1, 1, 1, 0, 0)
+                                   : conv_geom((uint64_t)height, (uint64_t)width, wo, (uint32_t)ksize, (uint32_t)ksize, (uint32_t)stride,
+                                               (int)(uint32_t)((uint64_t)pad - p0 / wo * (uint64_t)stride), pad);
+                if (!narrow) DKZ_TRY((launch_split<kSegWide, kTapWide>(kName, gj, 1)));
+                else if (ksize == 1 && kpos % 4 == 0) DKZ_TRY((launch_split<kSeg, kSeg>(kName, gj, 1)));
+                else if (ksize == 1) DKZ_TRY((launch_split<kSegOdd, kSegOdd>(kName, gj, 1)));
+                else if (kpos % 4 == 0) DKZ_TRY((launch_split<kSeg, kTap>(kName, gj, 1)));
+                else DKZ_TRY((launch_split<kSegOdd, kTap>(kName, gj, 1)));
+            }
         }
     }
     return 0;

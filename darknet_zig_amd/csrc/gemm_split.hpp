@@ -113,9 +113,11 @@ struct SplitArgs {
     ConvGeom cv;  // gathered operands and taps only
     // Weight gradient: positions per image, and those rounded up to a multiple
     // of four (k = image * kpos4 + position, so that four consecutive k lie in
-    // one image; the positions past kpos read as 0). a_img: delta's element
-    // stride from one image to the next; the input's is b_img.
-    uint32_t kpos;
+    // one image; the positions past kpos read as 0). krow: a row's elements (of
+    // delta, or of a 1x1 convolution's input), kpos but for a band of an image.
+    // a_img: delta's element stride from one image to the next; the input's is
+    // b_img.
+    uint32_t kpos, krow;
     uint64_t a_img;
     FastDiv div_kpos4;
     // phases != 0: grid row y runs phase y / zrows over group y % zrows, its
@@ -442,7 +444,7 @@ struct QuadBase {
     __device__ __forceinline__ bool tiny() const { return row.tiny(); }
 };
 
-// Rows of delta (row stride kpos): four positions in one 16-byte load. ODD: an
+// Rows of delta (row stride krow): four positions in one 16-byte load. ODD: an
 // image's last quad has fewer; it is loaded from kpos - 4 and shifted.
 template <int R, bool ODD>
 struct SegLoad : QuadBase<R> {
@@ -457,9 +459,9 @@ struct SegLoad : QuadBase<R> {
 #pragma unroll
         for (int l = 0; l < kL; ++l) {
             const uint32_t f = tid + l * kBlock, r = f / 4 < rows ? f / 4 : rows - 1;
-            at[l] = 4 * r * g.kpos;
+            at[l] = 4 * r * g.krow;
         }
-        buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + (size_t)img0 * img_stride + (size_t)r0 * g.kpos), 0,
+        buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + (size_t)img0 * img_stride + (size_t)r0 * g.krow), 0,
                                                 0x80000000u, 0x00020000);
     }
     __device__ __forceinline__ void load(uint32_t k0, uint32_t kend, int tid, uint64_t img_stride, const SplitArgs &g) {
@@ -527,7 +529,7 @@ struct TapLoad : QuadBase<R> {
     }
 };
 
-// Both with 64-bit addresses: img + r * kpos + p, and the tap's element.
+// Both with 64-bit addresses: img + r * krow + p, and the tap's element.
 template <int R, bool TAP>
 struct QuadWideLoad : QuadBase<R> {
     using QuadBase<R>::kL;
@@ -550,7 +552,7 @@ struct QuadWideLoad : QuadBase<R> {
                     ok = ok && y >= 0 && y < (int)cv.H && x >= 0 && x < (int)cv.W;
                     e += ((size_t)c * cv.H + y) * cv.W + x;
                 } else {
-                    e += (size_t)r * g.kpos + p;
+                    e += (size_t)r * g.krow + p;
                 }
                 ::dkz::lane(row.v[l], j) = ok ? base[e] : 0.0f;
             }

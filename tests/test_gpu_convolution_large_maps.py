@@ -47,12 +47,73 @@ def _case(batch, channels, H, W, filters, ks, stride, pad, nonzeros=20000):
     np.testing.assert_array_equal(got, want)
 
 
-@pytest.mark.parametrize("batch,H,W,ks", [(2, 4096, 4096, 1), (2, 4096, 4096, 3), (2, 5000, 5000, 3), (3, 2, 9000001, 1)])
+@pytest.mark.parametrize("batch,H,W,ks", [(2, 4096, 4096, 1), (2, 4096, 4096, 3), (2, 5000, 5000, 3), (3, 2, 9000001, 1),
+                                          (2, 9000001, 2, 3), (2, 1, 17000003, 3)])
 def test_positions_past_24_bits(dev, batch, H, W, ks):
-    """2^24 and more positions an image, in the second and third image too."""
+    """2^24 and more positions an image, in the second and third image too:
+    bands of rows, of positions (ksize 1), and 64-bit loaders (sides past 2^24)."""
     _case(batch, 1, H, W, 1, ks, 1, ks // 2)
+
+
+def test_bands_with_stride(dev):
+    _case(1, 1, 9001, 9003, 1, 3, 2, 1)  # 4501 x 4502 outputs: two bands
 
 
 def test_images_past_24_bits(dev):
     """2^24 + 5 images of one position."""
     _case((1 << 24) + 5, 1, 1, 1, 1, 3, 1, 1)
+
+
+def _sparse_case(batch, channels, H, W, filters, ks, stride, pad, at=24):
+    """Input and delta of zeros but for `at` positions of delta and the input's
+    windows there: tensors of gigabytes without their host copies."""
+    r = rng(batch + H + ks)
+    ho, wo = (H + 2 * pad - ks) // stride + 1, (W + 2 * pad - ks) // stride + 1
+    x, d = gpu.alloc(batch * channels * H * W), gpu.alloc(batch * filters * ho * wo)
+    dw = gpu.alloc(filters * channels * ks * ks)
+    values = {}  # the input's elements
+    def at_x(i, c, y, z):
+        return ((i * channels + c) * H + y) * W + z
+    try:
+        places = {(int(r.integers(batch)), int(r.integers(ho)), int(r.integers(wo))) for _ in range(at)}
+        places |= {(0, 0, 0), (batch - 1, ho - 1, wo - 1), (batch - 1, ho // 2, wo // 2)}
+        places = sorted(places)
+        for i, h, w in places:
+            z0, z1 = max(w * stride - pad, 0), min(w * stride - pad + ks, W)
+            for c in range(channels):
+                for y in range(max(h * stride - pad, 0), min(h * stride - pad + ks, H)):
+                    row = np.array([values.setdefault(at_x(i, c, y, z), int(r.integers(1, 9))) for z in range(z0, z1)], np.float32)
+                    gpu.push(x.offset(at_x(i, c, y, z0)), row)
+        want = np.zeros((filters, channels, ks, ks))
+        for i, h, w in places:
+            for f in range(filters):
+                v = int(r.integers(1, 9))
+                gpu.push(d.offset(((i * filters + f) * ho + h) * wo + w), np.array([v], np.float32))
+                for c in range(channels):
+                    for kh in range(ks):
+                        for kw in range(ks):
+                            y, z = h * stride + kh - pad, w * stride + kw - pad
+                            if 0 <= y < H and 0 <= z < W:
+                                want[f, c, kh, kw] += v * values[at_x(i, c, y, z)]
+        gpu.convolutionWeightGradient(batch, 1, channels, H, W, filters, ks, stride, pad, d, x, dw)
+        np.testing.assert_array_equal(down(dw, want.astype(np.float32)), want)
+    finally:
+        for b in (x, d, dw):
+            gpu.free(b)
+
+
+@pytest.mark.parametrize("case", [
+    # batch, channels, height, width, filters, ksize, stride, pad
+    (5, 8, 4000, 4000, 1, 3, 1, 1),     # 2.4 GiB of input: four images a product, then one
+    (3, 2, 4000, 4000, 16, 1, 1, 0),    # 2.9 GiB of delta: two images, then one
+    (40, 8, 1801, 1999, 2, 3, 2, 1),    # 4.3 GiB of input, odd maps: 18, 18 and 4 images
+    (1, 40, 3840, 3840, 3, 3, 1, 1),    # an image past 2^31 bytes: 64-bit addresses, K in ranges
+    (2, 1, 4095, 4097, 33, 1, 1, 0),    # the same in delta
+], ids=str)
+def test_batches_past_2_gib(dev, case):
+    _sparse_case(*case)
+
+
+def test_the_longest_map(dev):
+    """2^31 - 1 positions: rounded up to a multiple of four, 2^31."""
+    _sparse_case(1, 1, 1, 2**31 - 1, 1, 1, 1, 0)
