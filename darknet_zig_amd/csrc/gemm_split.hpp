@@ -5,7 +5,7 @@
 // bits each, rounded to nearest, so 24 bits in all): exact for |x| >= 2^-109.
 // A product of two such sums keeps six of its nine terms,
 //     hh | hm + mh + mm + hl + lh,
-// the rest being below 2^-25 of it. v_mfma_f32_32x32x16_bf16 forms the
+// the rest (ml, lm, ll) being up to 2^-24 of it, 2^-27.5 rms. v_mfma_f32_32x32x16_bf16 forms the
 // products exactly and adds them in fp32 with round to nearest. hh has an
 // accumulator of its own and the five small terms another, so the large one is
 // rounded once per 16 k (the fp32 matrix instruction rounds it at every k):
@@ -16,9 +16,8 @@
 // Where the split is not exact the tile is computed again with
 // v_mfma_f32_32x32x2_f32 from the same loads (redo): when an accumulator is
 // not finite (an infinity, a NaN, a value that rounds to a bf16 infinity: its
-// l is a NaN) or when all of a thread's share of some row is tiny (its largest
-// magnitude within (0, 2^-100)). Infinities, NaNs and tiny operands so give
-// what fp32 products give.
+// l is a NaN) or when any of the tile's operands lies within (0, 2^-109).
+// Infinities, NaNs and tiny operands so give what fp32 products give.
 //
 // A workgroup of four waves owns a BM x BN tile of C, each wave a quarter of
 // it. K advances in slabs of 16: each thread holds its share of the next slab
@@ -49,7 +48,6 @@ constexpr int kGroupM = 8;
 constexpr int kXcds = 8;
 constexpr int kPlanes = 3;
 constexpr int kF32Pitch = kBK + 4;  // LDS row pitch of the fp32 pass, in words
-constexpr float kTiny = 0x1p-100f;
 
 // LDS words of one half (8 k) of a plane of R rows, and of an operand's slab.
 template <int R>
@@ -175,23 +173,27 @@ __device__ __forceinline__ Split2 split2(float x, float y) {
     return s;
 }
 
-// Largest magnitude seen in one row's share; tiny() says the split loses bits.
-struct RowMax {
-    float mx = 0.0f;
-    __device__ __forceinline__ void see(float x, float y) { mx = fmaxf(fmaxf(mx, fabsf(x)), fabsf(y)); }
-    __device__ __forceinline__ bool tiny() const { return mx > 0.0f && mx < kTiny; }
+// Looks for values the split is not exact for: the smallest of 2|x| - 1, x taken
+// as its bits, in which zeros are the largest. (Three instructions a pair; the
+// largest magnitude of a row's share took one, but let a tiny value pass beside
+// a normal one, which is all of a sum where zeros lie opposite the normal ones.)
+struct Smallest {
+    uint32_t lo = ~0u;
+    static __device__ __forceinline__ uint32_t rank(float x) { return (__float_as_uint(x) << 1) - 1; }
+    __device__ __forceinline__ void see(float x, float y) { lo = min(min(lo, rank(x)), rank(y)); }
+    __device__ __forceinline__ bool tiny() const { return lo < rank(0x1p-109f); }
 };
 
 // ---- operand loaders: `load` takes a whole slab, `load_tail` one that ends at
 // kend (missing k read as 0); rows past the operand repeat its last row, whose
-// results are not stored. `store` writes the planes, `store_f32` the fp32 slab.
+// results are not stored. `store` writes the planes and shows `seen` the values,
+// `store_f32` writes the fp32 slab.
 
 template <int R>
 struct RowLoad {
     static constexpr int kL = R * kBK / 4 / kBlock;  // float4s per thread
     const float *p[kL];
     float4 v[kL];
-    RowMax mx[kL];
 
     __device__ __forceinline__ void init(const float *base, uint32_t ld, uint32_t r0, uint32_t rows, int tid) {
 #pragma unroll
@@ -215,13 +217,13 @@ struct RowLoad {
 #pragma unroll
             for (int j = 0; j < 4; ++j) ::dkz::lane(v[l], j) = kk + j < kend ? p[l][k0 + j] : 0.0f;
     }
-    __device__ __forceinline__ void store(uint32_t *s, int tid) {
+    __device__ __forceinline__ void store(uint32_t *s, int tid, Smallest &seen) const {
 #pragma unroll
         for (int l = 0; l < kL; ++l) {
             const int f = tid + l * kBlock, r = f / 4, q = f % 4;
             const Split2 x = split2(v[l].x, v[l].y), y = split2(v[l].z, v[l].w);
-            mx[l].see(v[l].x, v[l].y);
-            mx[l].see(v[l].z, v[l].w);
+            seen.see(v[l].x, v[l].y);
+            seen.see(v[l].z, v[l].w);
             uint32_t *d = s + (q >> 1) * half_words<R>() + r * 4 + (q & 1) * 2;
 #pragma unroll
             for (int u = 0; u < kPlanes; ++u)
@@ -235,12 +237,6 @@ struct RowLoad {
             *reinterpret_cast<float4 *>(s + (f / 4) * kF32Pitch + 4 * (f % 4)) = v[l];
         }
     }
-    __device__ __forceinline__ bool tiny() const {
-        bool t = false;
-#pragma unroll
-        for (int l = 0; l < kL; ++l) t |= mx[l].tiny();
-        return t;
-    }
 };
 
 // One row of the tile and kT consecutive k of each slab per thread: a wave's
@@ -250,15 +246,14 @@ template <int R>
 struct ColBase {
     static constexpr int kT = R * kBK / kBlock;
     float v[kT];
-    RowMax mx;
     uint32_t kq;  // wave-uniform: this wave's k start at kq * kT of the slab
 
-    __device__ __forceinline__ void store(uint32_t *s, int tid) {
+    __device__ __forceinline__ void store(uint32_t *s, int tid, Smallest &seen) const {
         Split2 w[kT / 2];
 #pragma unroll
         for (int j = 0; j < kT / 2; ++j) {
             w[j] = split2(v[2 * j], v[2 * j + 1]);
-            mx.see(v[2 * j], v[2 * j + 1]);
+            seen.see(v[2 * j], v[2 * j + 1]);
         }
         const int r = tid % R;
 #pragma unroll
@@ -275,7 +270,6 @@ struct ColBase {
 #pragma unroll
         for (int j = 0; j < kT; j += 4) *reinterpret_cast<float4 *>(d + j) = make_float4(v[j], v[j + 1], v[j + 2], v[j + 3]);
     }
-    __device__ __forceinline__ bool tiny() const { return mx.tiny(); }
 };
 
 template <int R>
@@ -438,10 +432,9 @@ struct Quad {
 template <int R>
 struct QuadBase {
     static constexpr int kL = RowLoad<R>::kL;
-    RowLoad<R> row;  // v and mx only
-    __device__ __forceinline__ void store(uint32_t *s, int tid) { row.store(s, tid); }
+    RowLoad<R> row;  // v only
+    __device__ __forceinline__ void store(uint32_t *s, int tid, Smallest &seen) const { row.store(s, tid, seen); }
     __device__ __forceinline__ void store_f32(float *s, int tid) const { row.store_f32(s, tid); }
-    __device__ __forceinline__ bool tiny() const { return row.tiny(); }
 };
 
 // Rows of delta (row stride krow): four positions in one 16-byte load. ODD: an
@@ -711,10 +704,11 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
             else sb[d].load_tail(k0, kend);
         }
     };
+    Smallest seen;
     auto store = [&](int d) {  // set d to LDS buffer d
         uint32_t *to = lds + d * (kA + kB);
-        sa[d].store(to, tid);
-        sb[d].store(to + kA, tid);
+        sa[d].store(to, tid, seen);
+        sb[d].store(to + kA, tid, seen);
     };
 
     f32x16 big[TM][TN], small[TM][TN];
@@ -796,9 +790,9 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
         __syncthreads();
     }
 
-    // Sum the accumulators; a value that is not finite, or a row whose share
-    // is tiny, sends the whole tile through the fp32 instruction.
-    bool redo = sa[0].tiny() || sa[1].tiny() || sb[0].tiny() || sb[1].tiny();
+    // Sum the accumulators; a value that is not finite, or a tiny operand,
+    // sends the whole tile through the fp32 instruction.
+    bool redo = seen.tiny();
 #pragma unroll
     for (int ti = 0; ti < TM; ++ti)
 #pragma unroll

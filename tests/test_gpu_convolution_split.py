@@ -80,3 +80,21 @@ def test_values_that_are_not_finite(dev, case, value):
         assert np.all(np.abs(got[fin] - want[fin]) <= bd[fin])
     for b in (dx, dw, dd, out, upd):
         gpu.free(b)
+
+
+def test_tiny_weights_beside_normal_ones(dev):
+    """Kernels whose centre tap alone meets the image (one pixel an image, the
+    other taps outside it): a centre of 2^-112 to 2^-140 beside taps near 1."""
+    case = (70, 1, 3, 1, 1, 29, 3, 1, 1)
+    batch, groups, C, H, W, F, ks, s, p = case
+    r = rng(6)
+    w = r.uniform(0.5, 1, (F, C, 9)).astype(np.float32)
+    w[:, :, 4] = np.ldexp(w[:, :, 4], -112 - np.arange(F)[:, None]).astype(np.float32)
+    x = np.ldexp(r.uniform(0.5, 1, batch * C), 40).astype(np.float32)
+    want, bd, _ = base._reference(case, x, w.ravel(), np.zeros(batch * F, np.float32))
+    dx, dw, out = up(x), up(w.ravel()), gpu.alloc(batch * F)
+    gpu.convolutionForward(batch, groups, C, H, W, F, ks, s, p, dw, dx, out)
+    got = down(out, np.empty(batch * F, np.float32)).astype(np.float64)
+    for b in (dx, dw, out):
+        gpu.free(b)
+    assert np.all(np.abs(got - want) <= bd)

@@ -94,6 +94,24 @@ def test_rows_of_many_scales(dev):
     check(np.ascontiguousarray(r.normal(size=(64, 64)).astype(np.float32)), np.ascontiguousarray(A.T))
 
 
+@pytest.mark.parametrize("ta,tb", VARIANTS)
+@pytest.mark.parametrize("side", ["A", "B"])
+def test_tiny_values_beside_normal_ones(dev, ta, tb, side):
+    """One tiny value a row, of every scale from 2^-95 to 2^-149, among normal
+    ones that meet zeros, so that it alone makes up the row's results."""
+    r = rng(12)
+    m, k, n = 165, 70, 64
+    A = r.normal(size=(m, k)).astype(np.float32)
+    B = np.zeros((k, n), np.float32)
+    at = 37
+    A[:, at] = np.ldexp(r.uniform(1, 2, m) * r.choice([-1, 1], m), -(95 + np.arange(m) % 55)).astype(np.float32)
+    B[at] = np.ldexp(r.uniform(1, 2, n), 60).astype(np.float32)
+    if side == "A":
+        check(A, B, ta, tb)
+    else:
+        check(np.ascontiguousarray(B.T), np.ascontiguousarray(A.T), ta, tb)
+
+
 def test_closer_to_f64_than_the_fp32_matrix_instruction(dev):
     """Rms error over K = 16 .. 4096 against the fp32 instruction's model (every
     product added with one rounding): no larger."""
