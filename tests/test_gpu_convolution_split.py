@@ -98,3 +98,26 @@ def test_tiny_weights_beside_normal_ones(dev):
     for b in (dx, dw, out):
         gpu.free(b)
     assert np.all(np.abs(got - want) <= bd)
+
+
+@pytest.mark.parametrize("case", [(42, 1, 75, 31, 31, 18, 1, 1, 0), (61, 1, 3, 19, 19, 23, 1, 1, 0), (9, 1, 6, 122, 122, 46, 3, 2, 1)], ids=str)
+def test_many_ranges_of_k_lose_nothing(dev, case):
+    """Weight gradients whose K is cut into a hundred ranges and more, positive
+    data. With u = 2^-24: the sum's one rounding leaves at most u, u / sqrt(3)
+    rms; a range of 20 slabs, rounded twice a slab at partial sums that grow to
+    the range's, at most sqrt(40 / 3) u / sqrt(3) rms, and a hundred independent
+    ranges a tenth of that: 0.62 u together. A fp32 sum of the ranges alone would
+    come to about sqrt(100 / 3) u / sqrt(3) = 3.3 u."""
+    batch, groups, C, H, W, F, ks, s, p = case
+    r = rng(8)
+    n = ref.conv_out_dim(H, ks, s, p) * ref.conv_out_dim(W, ks, s, p)
+    x = r.uniform(0.1, 1, batch * C * H * W).astype(np.float32)
+    d = r.uniform(0.1, 1, batch * F * n).astype(np.float32)
+    want, _ = base._wgrad_reference(case, x, d, np.zeros(F * C * ks * ks, np.float32))
+    dx, dd, upd = up(x), up(d), gpu.alloc(F * C * ks * ks)
+    gpu.convolutionWeightGradient(batch, groups, C, H, W, F, ks, s, p, dd, dx, upd)
+    got = down(upd, np.empty(want.size, np.float32)).astype(np.float64)
+    for b in (dx, dd, upd):
+        gpu.free(b)
+    rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert rel <= 0.62 * 2.0 ** -24, rel
