@@ -121,3 +121,19 @@ def test_many_ranges_of_k_lose_nothing(dev, case):
         gpu.free(b)
     rel = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert rel <= 0.62 * 2.0 ** -24, rel
+
+
+@pytest.mark.parametrize("ks", [1, 3, 5])
+def test_one_image_of_one_position_rounds_once(dev, ks):
+    """Weight gradients that are outer products: correctly rounded."""
+    r = rng(13)
+    C, F = 70, 40
+    x, d = r.normal(size=C).astype(np.float32), r.normal(size=F).astype(np.float32)
+    dx, dd, upd = up(x), up(d), gpu.alloc(F * C * ks * ks)
+    gpu.convolutionWeightGradient(1, 1, C, 1, 1, F, ks, 1, ks // 2, dd, dx, upd)
+    got = down(upd, np.empty(F * C * ks * ks, np.float32)).reshape(F, C, ks, ks)
+    for b in (dx, dd, upd):
+        gpu.free(b)
+    want = np.zeros_like(got)
+    want[:, :, ks // 2, ks // 2] = np.outer(d, x)
+    np.testing.assert_array_equal(got, want)

@@ -113,10 +113,10 @@ def test_tiny_values_beside_normal_ones(dev, ta, tb, side):
 
 
 def test_closer_to_f64_than_the_fp32_matrix_instruction(dev):
-    """Rms error over K = 16 .. 4096 against the fp32 instruction's model (every
+    """Rms error over K = 1 .. 4096 against the fp32 instruction's model (every
     product added with one rounding): no larger."""
     r = rng(9)
-    for k in (16, 256, 4096):
+    for k in (1, 2, 5, 16, 256, 4096):
         A, B = r.normal(size=(64, k)).astype(np.float32), r.normal(size=(k, 64)).astype(np.float32)
         want = A.astype(np.float64) @ B.astype(np.float64)
         chain = np.zeros((64, 64), np.float32)
@@ -124,3 +124,11 @@ def test_closer_to_f64_than_the_fp32_matrix_instruction(dev):
             chain = (chain.astype(np.float64) + np.outer(A[:, p].astype(np.float64), B[p].astype(np.float64))).astype(np.float32)
         err = np.linalg.norm(product(A, B) - want)
         assert err <= np.linalg.norm(chain - want), k
+
+
+@pytest.mark.parametrize("ta,tb", VARIANTS)
+def test_one_k_rounds_once(dev, ta, tb):
+    """An outer product is the correctly rounded one, bit for bit."""
+    r = rng(10)
+    A, B = r.normal(size=(130, 1)).astype(np.float32), r.normal(size=(1, 300)).astype(np.float32)
+    np.testing.assert_array_equal(product(A, B, ta, tb), A * B)
