@@ -150,18 +150,14 @@ int launch_split(const char *name, SplitArgs g, uint32_t z) {
                   : launch(name, stream_reduce_kernel<false>, blocks, block, g);
     }
     if (g.splits == 1) return 0;
-    const uint64_t mn = (uint64_t)g.m * g.n;
-    // Eight partials in flight; 32 where a small C has so many that their round
-    // trips would add up.
+    const uint64_t vecs = (uint64_t)g.m * g.n / (v4 ? 4 : 1);
     const bool many = g.splits > 32;
-    if (v4) {
-        const dim3 blocks(div_up(mn / 4, kBlock));
-        return many ? launch(name, split_reduce_kernel<true, 32>, blocks, block, g)
-                    : launch(name, split_reduce_kernel<true, 8>, blocks, block, g);
-    }
-    const dim3 blocks(div_up(mn, kBlock));
-    return many ? launch(name, split_reduce_kernel<false, 32>, blocks, block, g)
-                : launch(name, split_reduce_kernel<false, 8>, blocks, block, g);
+    const dim3 blocks(div_up(vecs, many ? kBlock / 16 : kBlock));
+    if (v4)
+        return many ? launch(name, split_reduce_kernel<true, 16>, blocks, block, g)
+                    : launch(name, split_reduce_kernel<true, 1>, blocks, block, g);
+    return many ? launch(name, split_reduce_kernel<false, 16>, blocks, block, g)
+                : launch(name, split_reduce_kernel<false, 1>, blocks, block, g);
 }
 
 // The data gradient's A: at[j][c][(f*ks + kh)*ks + kw] = w[j][f][c][ks-1-kh][ks-1-kw]

@@ -882,28 +882,48 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
 // kernel's own epilogue. The sum is kept in f64 and rounded once: with hundreds
 // of partials their fp32 sum was most of the error ([42,75,31,31]->18 1x1 weight
 // gradient: 4.5e-7 of the result with 255 partials in fp32, 0.7e-7 with 507 in
-// f64). V4: a
-// lane takes four consecutive columns of one row (one image's, 16-byte aligned).
-template <bool V4, int kReduceBatch>
+// f64). V4: a lane takes four consecutive columns of one row (one image's,
+// 16-byte aligned).
+//
+// GROUPS lanes share an output, lane g taking partials g, g + GROUPS, ..., and
+// the first adds the others' sums in order: one lane an output up to 32
+// partials, 16 beyond, where one lane's loads would take a round trip to memory
+// for every few partials ([1,50176]x[50176,9], 448 of them: 50 us with one lane,
+// 3.2 with 16).
+template <bool V4, int GROUPS>
 __global__ __launch_bounds__(kBlock) void split_reduce_kernel(SplitArgs g) {
     using T = std::conditional_t<V4, float4, float>;
-    constexpr uint32_t kW = V4 ? 4 : 1;
-    const uint32_t mn = g.m * g.n, v = blockIdx.x * kBlock + threadIdx.x;
-    if (v >= mn / kW) return;
-    const uint32_t e = v * kW, i = e / g.n, j = e - i * g.n;
-    // kReduceBatch partials in flight at a time; the missing ones of the last batch
-    // are +0, which leaves the sum as is.
+    constexpr uint32_t kW = V4 ? 4 : 1, kOuts = kBlock / GROUPS;
+    constexpr int kInFlight = 8;
+    const uint32_t mn = g.m * g.n, v = blockIdx.x * kOuts + threadIdx.x % kOuts, first = threadIdx.x / kOuts;
+    const bool in = v < mn / kW;
     double s[kW] = {};
-    for (uint32_t t = 0; t < g.splits; t += kReduceBatch) {
-        T p[kReduceBatch];
+    if (in) {
+        for (uint32_t t = first; t < g.splits; t += GROUPS * kInFlight) {
+            T p[kInFlight];  // past the last partial: that one again, not added
 #pragma unroll
-        for (int u = 0; u < kReduceBatch; ++u)
-            p[u] = t + u < g.splits ? reinterpret_cast<const T *>(g.partial + (size_t)(t + u) * mn)[v] : T{};
+            for (int u = 0; u < kInFlight; ++u)
+                p[u] = reinterpret_cast<const T *>(g.partial + (size_t)min(t + u * GROUPS, g.splits - 1) * mn)[v];
 #pragma unroll
-        for (int u = 0; u < kReduceBatch; ++u)
+            for (int u = 0; u < kInFlight; ++u)
 #pragma unroll
-            for (uint32_t x = 0; x < kW; ++x) s[x] += reinterpret_cast<const float *>(&p[u])[x];
+                for (uint32_t x = 0; x < kW; ++x)
+                    s[x] += t + u * GROUPS < g.splits ? (double)reinterpret_cast<const float *>(&p[u])[x] : 0.0;
+        }
     }
+    if constexpr (GROUPS > 1) {
+        __shared__ double sums[kW][kBlock];
+#pragma unroll
+        for (uint32_t x = 0; x < kW; ++x) sums[x][threadIdx.x] = s[x];
+        __syncthreads();
+        if (first != 0) return;
+#pragma unroll
+        for (int u = 1; u < GROUPS; ++u)
+#pragma unroll
+            for (uint32_t x = 0; x < kW; ++x) s[x] += sums[x][threadIdx.x + u * kOuts];
+    }
+    if (!in) return;
+    const uint32_t e = v * kW, i = e / g.n, j = e - i * g.n;
     float *cp = c_column(g.c, j, g, 0, 0) + (size_t)i * g.ldc;
     T o;
 #pragma unroll
@@ -929,15 +949,14 @@ __global__ __launch_bounds__(kBlock) void stream_reduce_kernel(SplitArgs g) {
     const float *from = g.partial + at + (size_t)t * tile_floats;
     double s[4] = {};
     for (uint32_t b = first; b <= last; b += kPieces) {
-        float4 p[kPieces];
+        float4 p[kPieces];  // past the last piece: that one again, not added
 #pragma unroll
         for (int u = 0; u < kPieces; ++u)
-            p[u] = b + u <= last ? *reinterpret_cast<const float4 *>(from + (size_t)(b + u) * tile_floats)
-                                 : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            p[u] = *reinterpret_cast<const float4 *>(from + (size_t)min(b + u, last) * tile_floats);
 #pragma unroll
         for (int u = 0; u < kPieces; ++u)
 #pragma unroll
-            for (int x = 0; x < 4; ++x) s[x] += ::dkz::lane(p[u], x);
+            for (int x = 0; x < 4; ++x) s[x] += b + u <= last ? (double)::dkz::lane(p[u], x) : 0.0;
     }
     if constexpr (V4) {
         float *cp = c_column(g.c, j, g, 0, 0) + (size_t)i * g.ldc;

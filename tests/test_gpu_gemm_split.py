@@ -55,6 +55,14 @@ def test_shapes(dev, ta, tb, m, n, k):
     check(r.normal(size=(m, k)).astype(np.float32), r.normal(size=(k, n)).astype(np.float32), ta, tb)
 
 
+@pytest.mark.parametrize("m,n,k", [(20, 64, 1000), (21, 65, 1000), (20, 64, 5000), (21, 65, 5000), (7, 12, 50000), (1, 9, 50176)])
+def test_k_in_ranges(dev, m, n, k):
+    """16, 79 and 448 partials, one and sixteen lanes an output, in float4s and
+    floats."""
+    r = rng(m + n + k)
+    check(r.normal(size=(m, k)).astype(np.float32), r.normal(size=(k, n)).astype(np.float32))
+
+
 @pytest.mark.parametrize("ta,tb", VARIANTS)
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, np.float32(3.4028235e38), np.float32(3.3961e38)])
 def test_values_the_split_cannot_hold(dev, ta, tb, value):
