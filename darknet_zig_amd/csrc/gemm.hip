@@ -542,6 +542,24 @@ int dkz_convolution_weight_gradient(int batch, int groups, int channels, int hei
     g.krow = (uint32_t)npos;
     g.a_img = (uint64_t)groups * m * npos;
     g.b_img = (uint64_t)groups * in_group;
+    constexpr const char *kName = "convolution_weight_gradient";
+    // One position an image (a classifier's 1x1 layer behind a global average
+    // pool): images are rows of delta and input, a plain TN product whose k are
+    // the images. [256,2048,1,1]->1000 43.5 us on the fp32 instruction, 54.8
+    // through the 64-bit quad loaders, which pad its k to four, 14.0 so.
+    if (npos == 1 && ksize == 1) {
+        g.k = (uint32_t)batch;
+        g.lda = (uint32_t)g.a_img;
+        g.ldb = (uint32_t)g.b_img;
+        for (int j = 0; j < groups; ++j) {
+            SplitArgs gj = g;
+            gj.a = delta + (uint64_t)j * m;
+            gj.b = input + (uint64_t)j * in_group;
+            gj.c = weight_updates + (uint64_t)j * m * kw;
+            DKZ_TRY((launch_split<kColMajor, kColMajor>(kName, gj, 1)));
+        }
+        return 0;
+    }
     // The narrow loaders: an image within 2^31 bytes, at least one whole quad
     // an image, and 24-bit products: a map of 2^24 positions or more goes
     // through them in bands of output rows (of positions, where ksize 1 reads
@@ -563,7 +581,6 @@ int dkz_convolution_weight_gradient(int batch, int groups, int channels, int hei
     uint64_t most = std::min<uint64_t>((uint64_t)batch, std::max<uint64_t>(kMaxElems / up4(band), 1));
     if (narrow) most = std::min({most, k24 - 1, (kMaxOffset - 1) / img_bytes});
     if (bands > 1) most = 1;
-    constexpr const char *kName = "convolution_weight_gradient";
     for (int j = 0; j < groups; ++j) {
         for (uint64_t i0 = 0; i0 < (uint64_t)batch; i0 += most) {
             for (uint64_t p0 = 0; p0 < npos; p0 += band) {

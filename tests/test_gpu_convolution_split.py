@@ -52,6 +52,15 @@ def test_data_gradient(dev, case):
     base.test_convolution_data_gradient(dev, case)
 
 
+@pytest.mark.parametrize("case", [(150, 2, 6, 1, 1, 70, 1, 1, 0), (5, 1, 130, 2, 3, 65, 1, 3, 0), (700, 1, 40, 1, 1, 33, 1, 1, 0),
+                                  (300, 1, 5, 1, 2, 9, 1, 1, 0), (130, 2, 6, 3, 1, 4, 3, 1, 1)], ids=str)
+def test_weight_gradient_of_one_to_three_positions(dev, case):
+    """One position with ksize 1 is a TN product over the images (also of an
+    image larger than the positions read); the others take 64-bit quads, K in
+    ranges."""
+    base.test_convolution_weight_gradient(dev, case)
+
+
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
 @pytest.mark.parametrize("case", [(2, 1, 8, 9, 9, 40, 3, 1, 1), (2, 1, 8, 8, 8, 40, 1, 1, 0)], ids=str)
 def test_values_that_are_not_finite(dev, case, value):
