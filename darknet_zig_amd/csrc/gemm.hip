@@ -224,9 +224,14 @@ ConvGeom conv_geom(uint64_t H, uint64_t W, uint64_t wo, uint32_t rows, uint32_t 
 
 // A product whose B is gathered from images of `in_group` elements each.
 int launch_gather(const char *name, const SplitArgs &g, uint32_t z, uint64_t in_group) {
-    bool narrow = g.cv.rows <= 32 && g.cv.cols <= 32 &&
-                  span_fits(g.npos, g.b_img, in_group + (uint64_t)g.cv.rows * g.cv.W + g.cv.cols);
-    for (uint32_t p = 0; p < g.phases; ++p) narrow = narrow && g.ph[p].rows <= 32 && g.ph[p].cols <= 32;
+    // kGather's offsets count from a window's first tap at position (0, 0), so
+    // the image's last element lies pad rows and pad_x elements further on.
+    const auto fits = [&](uint32_t rows, uint32_t cols, int pad, int pad_x) {
+        return rows <= 32 && cols <= 32 &&
+               span_fits(g.npos, g.b_img, in_group + (uint64_t)std::max(pad, 0) * g.cv.W + (uint64_t)std::max(pad_x, 0));
+    };
+    bool narrow = fits(g.cv.rows, g.cv.cols, g.cv.pad, g.cv.pad_x);
+    for (uint32_t p = 0; p < g.phases; ++p) narrow = narrow && fits(g.ph[p].rows, g.ph[p].cols, g.ph[p].pad, g.ph[p].pad_x);
     return narrow ? launch_split<kRowMajor, kGather>(name, g, z) : launch_split<kRowMajor, kGatherWide>(name, g, z);
 }
 

@@ -1,6 +1,5 @@
-"""Convolution weight gradients over maps so large, or batches so long, that the
-product kernel's narrow loaders (24-bit products, 32-bit byte offsets) do not
-take them. Inputs are small integers and delta is sparse, so every summation
+"""Convolutions over maps so large, or batches so long, that the product kernel's
+narrow loaders (24-bit products, 32-bit byte offsets) do not take them. Inputs are small integers and delta is sparse, so every summation
 order is exact and the results must match bit for bit."""
 
 from __future__ import annotations
@@ -117,3 +116,31 @@ def test_batches_past_2_gib(dev, case):
 def test_the_longest_map(dev):
     """2^31 - 1 positions: rounded up to a multiple of four, 2^31."""
     _sparse_case(1, 1, 1, 2**31 - 1, 1, 1, 1, 0)
+
+
+def test_forward_with_padding_past_2_gib(dev):
+    """An image of 0.8 GB and padding larger than the window: from a window's
+    first tap at (0, 0) the image's last rows lie past 2^31 bytes."""
+    H, W, ks, stride, pad = 1000, 200000, 3, 16, 1700
+    ho, wo = (H + 2 * pad - ks) // stride + 1, (W + 2 * pad - ks) // stride + 1
+    r = rng(3)
+    w = r.integers(1, 9, (ks, ks)).astype(np.float32)
+    want = np.zeros((ho, wo), np.float32)
+    x, dw, out = gpu.alloc(H * W), up(w.ravel()), gpu.alloc(ho * wo)
+    try:
+        taps = {(int(h), int(q), int(kh), int(kw)) for h, q, kh, kw in
+                zip(r.integers(107, 168, 60), r.integers(107, 12606, 60), r.integers(0, ks, 60), r.integers(0, ks, 60))}
+        placed = {}
+        for h, q, kh, kw in taps | {(168, 12606, 0, 0), (168, 12605, 1, 2)}:
+            y, z = h * stride + kh - pad, q * stride + kw - pad
+            if 0 <= y < H and 0 <= z < W:
+                placed[y, z] = (h, q, kh, kw, float(r.integers(1, 9)))
+        assert max(y for y, _ in placed) > 980
+        for (y, z), (h, q, kh, kw, v) in placed.items():  # strides past the window: one output each
+            gpu.push(x.offset(y * W + z), np.array([v], np.float32))
+            want[h, q] += v * w[kh, kw]
+        gpu.convolutionForward(1, 1, 1, H, W, 1, ks, stride, pad, dw, x, out)
+        np.testing.assert_array_equal(down(out, want), want)
+    finally:
+        for b in (x, dw, out):
+            gpu.free(b)
