@@ -19,7 +19,7 @@ void set_error_context(const char *fmt, ...);
 // Called right after a kernel launch: reports a launch error, and under
 // sync-after-launch waits for the kernel and reports its fault. `name` and the
 // launch shape go into the error context (gpu.zig:445-462).
-int after_launch(const char *name, dim3 grid, dim3 block);
+int after_launch(const char *name, dim3 grid, dim3 block, hipStream_t stream = current_stream());
 
 // Whether sync-after-launch is on (DARKNET_GPU_SYNC, dkz_set_sync_after_launch).
 bool sync_after_launch();
@@ -55,10 +55,14 @@ bool recently_written(const void *p, uint64_t bytes);
 void batchnorm_prewarm();
 
 template <typename Kernel, typename... Args>
-inline int launch(const char *name, Kernel kernel, dim3 grid, dim3 block, Args... args) {
+inline int launch_on(hipStream_t stream, const char *name, Kernel kernel, dim3 grid, dim3 block, Args... args) {
     (void)hipGetLastError();  // a stale error from the caller's own calls is not ours
-    hipLaunchKernelGGL(kernel, grid, block, 0, current_stream(), args...);
-    return after_launch(name, grid, block);
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, args...);
+    return after_launch(name, grid, block, stream);
+}
+template <typename Kernel, typename... Args>
+inline int launch(const char *name, Kernel kernel, dim3 grid, dim3 block, Args... args) {
+    return launch_on(current_stream(), name, kernel, grid, block, args...);
 }
 
 // Devices the library keeps per-device state for (ordinals 0..63).
@@ -84,6 +88,9 @@ constexpr uint32_t kScratchPartials = 1u << 18;    // channels * chunks (2 MiB o
 #endif
 constexpr uint64_t kScratchGemmFloats = 1ull << DKZ_SCRATCH_GEMM_LOG2;  // split-K partial tiles (128 MiB)
 constexpr uint32_t kScratchSlots = 1u << 16;         // 64-bit counter slots (512 KiB)
+// The null stream's block for products that must not share the partial tiles
+// above: the pieces of one streamed round of 128x128 tiles at most (64 MiB).
+constexpr uint64_t kScratchOwnFloats = 1ull << 24;
 // A split reduction's per-channel counters and f64 partials sit
 // kCounterStride / kPartialStride elements apart, so that no two share a
 // 128-byte line: atomics and write-through stores to one line are
@@ -97,6 +104,9 @@ constexpr uint32_t kScratchSlots = 1u << 16;         // 64-bit counter slots (51
 constexpr uint32_t kCounterStride = DKZ_SPLIT_CSTRIDE;
 constexpr uint32_t kPartialStride = DKZ_SPLIT_PSTRIDE;
 int device_scratch(Scratch *out);
+// The current device's null-stream block, null where the device has no scratch
+// yet (allocates nothing).
+float *null_stream_scratch();
 
 // While one of these lives, device_scratch() on this host thread returns
 // *s instead of the library's allocated scratch (and allocates nothing): the

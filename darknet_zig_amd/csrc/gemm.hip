@@ -18,6 +18,7 @@
 // one XCD (workgroups are dealt to the 8 XCDs round robin) so that they share
 // its L2.
 #include <algorithm>
+#include <mutex>
 #include <vector>
 
 #include "dkz_device.hpp"
@@ -104,20 +105,63 @@ Tiling pick_tiling(uint64_t m, uint64_t n, uint64_t k, uint64_t z, uint64_t max_
     return best;
 }
 
-// Runs a product of g's operands over `z` grid rows (one when K may be split).
+// Held from a null-stream product's launch to its reduction's (see launch_split).
+std::mutex g_own_mutex;
+
 template <Operand AK, Operand BK>
+int launch_tiles(hipStream_t stream, const char *name, uint32_t bm, uint32_t bn, dim3 grid, const SplitArgs &g) {
+    const dim3 block(kBlock);
+    if constexpr (BK != kGatherWide && BK != kTapWide) {
+        if (bm == 128 && bn == 128) return launch_on(stream, name, gemm_split_kernel<128, 128, AK, BK>, grid, block, g);
+        if (bm == 128) return launch_on(stream, name, gemm_split_kernel<128, 64, AK, BK>, grid, block, g);
+        if (bm == 64 && bn == 128) return launch_on(stream, name, gemm_split_kernel<64, 128, AK, BK>, grid, block, g);
+        if (bm == 32) return launch_on(stream, name, gemm_split_kernel<32, 128, AK, BK>, grid, block, g);
+    }
+    return launch_on(stream, name, gemm_split_kernel<64, 64, AK, BK>, grid, block, g);
+}
+
+// The tiles from full_tiles on, a workgroup taking all of a tile's pieces.
+template <Operand AK, Operand BK>
+int launch_ordered(hipStream_t stream, const char *name, const SplitArgs &g) {
+    const uint32_t tiles = g.tiles_m * g.tiles_n - g.full_tiles;
+    const dim3 block(kBlock);
+    if constexpr (BK != kGatherWide)
+        if (g.tile_bm == 32) return launch_on(stream, name, gemm_split_kernel<32, 128, AK, BK, true>, dim3(tiles), block, g);
+    const dim3 grid(tiles * (g.tile_bm / 64) * ((1u << g.tile_bn_log2) / 64));
+    return launch_on(stream, name, gemm_split_kernel<64, 64, AK, BK, true>, grid, block, g);
+}
+
+// Runs a product of g's operands over `z` grid rows (one when K may be split).
+//
+// The partials of K ranges and pieces go to g.partial, in the device's scratch
+// (null: K is not split), which calls on several streams must not share at the
+// same time. OWN: a product of which calls may overlap on any streams, threads
+// and captured graphs (a convolution's forward, its 1x1 data gradient). On the
+// null stream, where calls run one behind the other, its partials have a block
+// of the scratch to themselves, and a mutex keeps another thread's product from
+// between a product and its reduction; on other streams a workgroup takes all of
+// a tile's pieces itself (launch_ordered), with the same results. Null stream /
+// another, us, and the unsplit fp32 kernel this replaced: [1,64,52,52]->128 3x3
+// 16.8 / 25.5 / 38; [64,128,56,56]->128 367 / 402 / 688; [32,512,13,13]->1024 337 /
+// 482 / 622; [1,512,13,13]->1024 28 / 146 / 249, where 48 tiles leave most CUs idle.
+template <Operand AK, Operand BK, bool OWN = false>
 int launch_split(const char *name, SplitArgs g, uint32_t z) {
     uint64_t max_splits = 0, left = 0;
-    Scratch sc{};
-    if (z == 1 && g.phases == 0 && g.partial != nullptr && g.k >= 8 * kBK) {
-        DKZ_TRY(device_scratch(&sc));
-        left = (uint64_t)(sc.gemm + sc.gemm_floats - g.partial);
+    if (z == 1 && g.phases == 0 && g.k >= 8 * kBK && (OWN || g.partial != nullptr)) {
+        if constexpr (OWN) {
+            left = kScratchOwnFloats;
+        } else {
+            Scratch sc{};
+            DKZ_TRY(device_scratch(&sc));
+            left = (uint64_t)(sc.gemm + sc.gemm_floats - g.partial);
+        }
         max_splits = std::max<uint64_t>(1, std::min<uint64_t>(kMaxSplits, left / ((uint64_t)g.m * g.n)));
     }
-    constexpr bool kWide = BK == kGatherWide || BK == kTapWide;
-    const Tiling t = pick_tiling(g.m, g.n, g.k, z, max_splits, left, kWide);
+    const Tiling t = pick_tiling(g.m, g.n, g.k, z, max_splits, left, BK == kGatherWide || BK == kTapWide);
     g.tiles_m = div_up(g.m, t.bm);
     g.tiles_n = div_up(g.n, t.bn);
+    g.tile_bm = t.bm;
+    g.tile_bn_log2 = t.bn == 128 ? 7 : 6;
     g.splits = t.splits;
     g.k_chunk = t.k_chunk;
     uint64_t total = (uint64_t)g.tiles_m * g.tiles_n * g.splits;
@@ -128,36 +172,38 @@ int launch_split(const char *name, SplitArgs g, uint32_t z) {
         g.stream_len = t.stream;
         g.stream_slabs = streamed * slabs;
         g.div_tile_slabs = make_fastdiv(slabs);
-        g.tile_bm = t.bm;
-        g.tile_bn_log2 = t.bn == 128 ? 7 : 6;
         total = t.full_tiles + div_up(g.stream_slabs, t.stream);
     }
     DKZ_REQUIRE(total <= 0x7fffffffull);
-    const dim3 grid((uint32_t)total, z), block(kBlock);
-    if constexpr (kWide) {
-        DKZ_TRY(launch(name, gemm_split_kernel<64, 64, AK, BK>, grid, block, g));
-    } else {
-        if (t.bm == 128 && t.bn == 128) DKZ_TRY(launch(name, gemm_split_kernel<128, 128, AK, BK>, grid, block, g));
-        else if (t.bm == 128) DKZ_TRY(launch(name, gemm_split_kernel<128, 64, AK, BK>, grid, block, g));
-        else if (t.bm == 64 && t.bn == 128) DKZ_TRY(launch(name, gemm_split_kernel<64, 128, AK, BK>, grid, block, g));
-        else if (t.bm == 32) DKZ_TRY(launch(name, gemm_split_kernel<32, 128, AK, BK>, grid, block, g));
-        else DKZ_TRY(launch(name, gemm_split_kernel<64, 64, AK, BK>, grid, block, g));
+    const hipStream_t stream = current_stream();
+    std::unique_lock<std::mutex> lock(g_own_mutex, std::defer_lock);
+    if constexpr (OWN) {
+        if (t.stream || g.splits > 1) {
+            g.partial = stream == nullptr ? null_stream_scratch() : nullptr;
+            if (g.partial == nullptr) {
+                if (g.full_tiles != 0) DKZ_TRY((launch_tiles<AK, BK>(stream, name, t.bm, t.bn, dim3(g.full_tiles), g)));
+                return launch_ordered<AK, BK>(stream, name, g);
+            }
+            lock.lock();
+        }
     }
+    DKZ_TRY((launch_tiles<AK, BK>(stream, name, t.bm, t.bn, dim3((uint32_t)total, z), g)));
     const bool v4 = g.n % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.c) && g.npos % 4 == 0 && g.c_img % 4 == 0;
+    const dim3 block(kBlock);
     if (t.stream) {
         const dim3 blocks(streamed * (t.bm * t.bn / 4 / kBlock));
-        return v4 ? launch(name, stream_reduce_kernel<true>, blocks, block, g)
-                  : launch(name, stream_reduce_kernel<false>, blocks, block, g);
+        return v4 ? launch_on(stream, name, stream_reduce_kernel<true>, blocks, block, g)
+                  : launch_on(stream, name, stream_reduce_kernel<false>, blocks, block, g);
     }
     if (g.splits == 1) return 0;
     const uint64_t vecs = (uint64_t)g.m * g.n / (v4 ? 4 : 1);
     const bool many = g.splits > 32;
     const dim3 blocks(div_up(vecs, many ? kBlock / 16 : kBlock));
     if (v4)
-        return many ? launch(name, split_reduce_kernel<true, 16>, blocks, block, g)
-                    : launch(name, split_reduce_kernel<true, 1>, blocks, block, g);
-    return many ? launch(name, split_reduce_kernel<false, 16>, blocks, block, g)
-                : launch(name, split_reduce_kernel<false, 1>, blocks, block, g);
+        return many ? launch_on(stream, name, split_reduce_kernel<true, 16>, blocks, block, g)
+                    : launch_on(stream, name, split_reduce_kernel<true, 1>, blocks, block, g);
+    return many ? launch_on(stream, name, split_reduce_kernel<false, 16>, blocks, block, g)
+                : launch_on(stream, name, split_reduce_kernel<false, 1>, blocks, block, g);
 }
 
 // The data gradient's A: at[j][c][(f*ks + kh)*ks + kw] = w[j][f][c][ks-1-kh][ks-1-kw]
@@ -223,6 +269,7 @@ ConvGeom conv_geom(uint64_t H, uint64_t W, uint64_t wo, uint32_t rows, uint32_t 
 }
 
 // A product whose B is gathered from images of `in_group` elements each.
+template <bool OWN>
 int launch_gather(const char *name, const SplitArgs &g, uint32_t z, uint64_t in_group) {
     // kGather's offsets count from a window's first tap at position (0, 0), so
     // the image's last element lies pad rows and pad_x elements further on.
@@ -232,7 +279,7 @@ int launch_gather(const char *name, const SplitArgs &g, uint32_t z, uint64_t in_
     };
     bool narrow = fits(g.cv.rows, g.cv.cols, g.cv.pad, g.cv.pad_x);
     for (uint32_t p = 0; p < g.phases; ++p) narrow = narrow && fits(g.ph[p].rows, g.ph[p].cols, g.ph[p].pad, g.ph[p].pad_x);
-    return narrow ? launch_split<kRowMajor, kGather>(name, g, z) : launch_split<kRowMajor, kGatherWide>(name, g, z);
+    return narrow ? launch_split<kRowMajor, kGather, OWN>(name, g, z) : launch_split<kRowMajor, kGatherWide, OWN>(name, g, z);
 }
 
 // Extent in elements of a rows x cols row-major view with leading dimension ld.
@@ -305,8 +352,6 @@ int dkz_convolution_forward(int batch, int groups, int channels, int height, int
     DKZ_REQUIRE(weights && input && output);
     DKZ_REQUIRE(zcount * m * n <= kMaxElems && zcount * in_group <= kMaxElems && (uint64_t)groups * m * k <= kMaxElems);
     DKZ_REQUIRE(ksize != 1 || n <= (uint64_t)height * width);  // the input is read as a k x n matrix
-    Scratch sc;
-    DKZ_TRY(device_scratch(&sc));
     SplitArgs g{};
     g.a = weights;
     g.b = input;
@@ -318,18 +363,18 @@ int dkz_convolution_forward(int batch, int groups, int channels, int height, int
     g.ldc = (uint32_t)n;
     g.alpha = 1.0f;
     g.beta = 1.0f;
-    g.partial = sc.gemm;
     g.zgroups = (uint32_t)groups;
     g.a_z = m * k;
     g.b_z = in_group;
     g.c_z = m * n;
     set_span(g, n, (uint64_t)batch, (uint64_t)groups * in_group, (uint64_t)groups * m * n);
     constexpr const char *kName = "convolution_forward";
-    if (ksize == 1 && span_fits(n, g.b_img, 0)) return launch_split<kRowMajor, kColMajor>(kName, g, (uint32_t)groups);
+    if (ksize == 1 && span_fits(n, g.b_img, 0)) 
+        return launch_split<kRowMajor, kColMajor, true>(kName, g, (uint32_t)groups);
     // ksize 1 reads the input as a k x n matrix: rows of n positions.
     g.cv = ksize == 1 ? conv_geom(1, n, n, 1, 1, 1, 0, 0)
                       : conv_geom((uint64_t)height, (uint64_t)width, wo, (uint32_t)ksize, (uint32_t)ksize, (uint32_t)stride, pad, pad);
-    return launch_gather(kName, g, (uint32_t)groups, in_group);
+    return launch_gather<true>(kName, g, (uint32_t)groups, in_group);
 }
 
 // convolutional.zig:299-305 (the data-gradient half of the per-image
@@ -365,14 +410,11 @@ int dkz_convolution_data_gradient(int batch, int groups, int channels, int heigh
     DKZ_REQUIRE(zcount * m * npos <= kMaxElems && zcount * in_group <= kMaxElems &&
                 (uint64_t)groups * m * kw <= kMaxElems);
     DKZ_REQUIRE(ksize != 1 || npos <= (uint64_t)height * width);  // the k x n view stays inside the image
-    Scratch sc;
-    DKZ_TRY(device_scratch(&sc));
     SplitArgs g{};
     g.c = input_delta;
     g.b = delta;
     g.m = (uint32_t)cg;
     g.alpha = 1.0f;
-    g.partial = sc.gemm;
     g.zgroups = (uint32_t)groups;
     g.b_z = m * npos;
     g.c_z = in_group;
@@ -389,11 +431,13 @@ int dkz_convolution_data_gradient(int batch, int groups, int channels, int heigh
         g.beta = 0.0f;
         g.a_z = m * cg;
         set_span(g, npos, (uint64_t)batch, b_img, c_img);
-        if (span_fits(npos, b_img, 0)) return launch_split<kColMajor, kColMajor>(kName, g, (uint32_t)groups);
+        if (span_fits(npos, b_img, 0)) return launch_split<kColMajor, kColMajor, true>(kName, g, (uint32_t)groups);
         g.cv = conv_geom(1, npos, npos, 1, 1, 1, 0, 0);
-        return launch_split<kColMajor, kGatherWide>(kName, g, (uint32_t)groups);
+        return launch_split<kColMajor, kGatherWide, true>(kName, g, (uint32_t)groups);
     }
     if (m == 0) return 0;  // col2im adds an empty sum
+    Scratch sc;
+    DKZ_TRY(device_scratch(&sc));
     g.beta = 1.0f;
     if (stride == 1 && pad <= ksize - 1) {
         // input_delta(i, j) += A x im2col(delta(i, j)) with A the group's
@@ -419,7 +463,7 @@ int dkz_convolution_data_gradient(int batch, int groups, int channels, int heigh
         set_span(g, n, (uint64_t)batch, b_img, c_img);
         const int back = ksize - 1 - pad;
         g.cv = conv_geom(ho, wo, (uint64_t)width, (uint32_t)ksize, (uint32_t)ksize, 1, back, back);
-        return launch_gather(kName, g, (uint32_t)groups, m * npos);
+        return launch_gather<false>(kName, g, (uint32_t)groups, m * npos);
     }
     // Strided (or pad >= ksize): the im2col of delta would have holes between
     // the strided outputs. Input pixel (y, x) takes tap (kh, kw) only when
@@ -503,7 +547,7 @@ int dkz_convolution_data_gradient(int batch, int groups, int channels, int heigh
         gp.div_wp = make_fastdiv((uint32_t)wp);
         set_span(gp, n, (uint64_t)batch, b_img, c_img);
         gp.cv = conv_geom(ho, wo, (uint64_t)wp, gp.ph[0].rows, gp.ph[0].cols, 1, gp.ph[0].pad, gp.ph[0].pad_x);
-        DKZ_TRY(launch_gather(kName, gp, (uint32_t)(cnt * groups), m * npos));
+        DKZ_TRY(launch_gather<false>(kName, gp, (uint32_t)(cnt * groups), m * npos));
         i0 += cnt;
     }
     return 0;

@@ -596,8 +596,13 @@ template <int R> struct Loader<kTapWide, R> { using type = QuadWideLoad<R, true>
 template <int BM, int BN>
 constexpr int min_waves() { return BM * BN >= 128 * 128 ? 2 : BM * BN >= 128 * 64 ? 3 : 4; }
 
-template <int BM, int BN, Operand AK, Operand BK>
-__global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kernel(SplitArgs g) {
+// ORDERED: a workgroup takes all of a tile's K ranges or pieces, one behind the
+// other, and keeps their sum in f64 as the reductions do, so that no scratch is
+// needed and the results are the same. Tiles are 64x64 (their sums take 32
+// registers; a 128x128 tile's would take 128), each a part of the g.tile_bm x
+// g.tile_bn tile whose pieces it adds up, or the 32x128 ones.
+template <int BM, int BN, Operand AK, Operand BK, bool ORDERED = false>
+__global__ __launch_bounds__(kBlock, (min_waves<BM, BN>() - (ORDERED ? 1 : 0))) void gemm_split_kernel(SplitArgs g) {
     constexpr int kRowsOfWaves = BM == 32 ? 1 : 2;  // 32-row tiles: four waves side by side
     constexpr int WM = BM / kRowsOfWaves, WN = BN * kRowsOfWaves / 4, TM = WM / 32, TN = WN / 32;
     constexpr int RA = BM == 32 ? 64 : BM;  // rows of A staged (of a 32-row tile, the last row again)
@@ -643,9 +648,25 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
     // One K range of one tile; or a run of the streamed line: the last slabs of
     // a tile, the first ones of the next. Piece (workgroup b, tile t) has
     // partial tile b + t (along the line at least one of the two advances).
-    const bool streams = g.stream_len != 0 && blockIdx.x >= g.full_tiles;
-    uint32_t block = blockIdx.x, line = 0, line_end = 0;
-    if (streams) {
+    const bool streams = !ORDERED && g.stream_len != 0 && blockIdx.x >= g.full_tiles;
+    uint32_t block = blockIdx.x, line = 0, line_end = 0, run = 0;
+    [[maybe_unused]] double total[ORDERED ? TM : 1][ORDERED ? TN : 1][ORDERED ? 16 : 1] = {};
+    [[maybe_unused]] uint32_t own_m0 = 0, own_n0 = 0;
+    if constexpr (ORDERED) {  // the tile's slabs along the line, or from 0; cut at multiples of run
+        const uint32_t subs_n = g.tile_bn_log2 == 7 && BN == 64 ? 2 : 1, subs = subs_n * (g.tile_bm == 128 ? 2 : 1);
+        block = xcd_order(block, (g.tiles_m * g.tiles_n - g.full_tiles) * subs);
+        const uint32_t sub = block % subs;
+        block /= subs;
+        uint32_t tm, tn;
+        tile_at(g.full_tiles + block, g, tm, tn);
+        own_m0 = tm * g.tile_bm + sub / subs_n * BM;
+        own_n0 = (tn << g.tile_bn_log2) + sub % subs_n * BN;
+        if (own_m0 >= g.m || own_n0 >= g.n) return;
+        const uint32_t slabs = (k_all + kBK - 1) / kBK;
+        run = g.stream_len != 0 ? g.stream_len : k_chunk / kBK;
+        line = g.stream_len != 0 ? block * slabs : 0;
+        line_end = line + slabs;
+    } else if (streams) {
         block = xcd_order(block - g.full_tiles, gridDim.x - g.full_tiles);
         line = block * g.stream_len;
         line_end = min(line + g.stream_len, g.stream_slabs);
@@ -653,7 +674,13 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
 #pragma unroll 1
     do {
     uint32_t tm, tn, kbeg, kend, slot = 0;
-    if (streams) {
+    if constexpr (ORDERED) {
+        const uint32_t len = min(run - line % run, line_end - line);
+        tm = tn = 0;
+        kbeg = (line + (k_all + kBK - 1) / kBK - line_end) * kBK;
+        kend = min(kbeg + len * kBK, k_all);
+        line += len;
+    } else if (streams) {
         const uint32_t t = fdiv(line, g.div_tile_slabs), first = line - t * g.div_tile_slabs.d;
         const uint32_t len = min(g.div_tile_slabs.d - first, line_end - line);
         tile_at(g.full_tiles + t, g, tm, tn);
@@ -669,7 +696,7 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
         kbeg = slot * k_chunk;
         kend = kbeg + k_chunk < k_all ? kbeg + k_chunk : k_all;
     }
-    const uint32_t m0 = tm * BM, n0 = tn * BN;
+    const uint32_t m0 = ORDERED ? own_m0 : tm * BM, n0 = ORDERED ? own_n0 : tn * BN;
 
     // Two register sets: slab s is loaded into set s & 1.
     typename Loader<AK, RA>::type sa[2];
@@ -833,6 +860,22 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
         }
     }
 
+    if constexpr (ORDERED) {
+#pragma unroll
+        for (int ti = 0; ti < TM; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < TN; ++tj)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) total[ti][tj][r] += (double)big[ti][tj][r];
+        if (line < line_end) continue;
+#pragma unroll
+        for (int ti = 0; ti < TM; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < TN; ++tj)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) big[ti][tj][r] = (float)total[ti][tj][r];
+    }
+
     // big[ti][tj][r] is C(row, col) of the wave's block (ti, tj) with
     // row = 8*(r/4) + 4*(lane/32) + r%4 and col = lane%32. A block's sixteen
     // values of C are loaded together (rows past m read row m - 1), then stored.
@@ -846,7 +889,7 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>())) void gemm_split_kern
             const uint32_t i0 = m0 + wm0 + ti * 32 + half * 4;
             const auto row = [&](int r) { return i0 + (r >> 2) * 8 + (r & 3); };
             // A K range's partial is a whole m x n one, a streamed piece's its tile.
-            const bool part = streams || g.splits > 1;
+            const bool part = !ORDERED && (streams || g.splits > 1);
             float *to = !part     ? ccol
                         : streams ? g.partial + (size_t)slot * (BM * BN) + (j - n0) - (size_t)m0 * BN
                                   : g.partial + (size_t)slot * g.m * g.n + j;

@@ -44,7 +44,8 @@ bool env_flag(const char *name) {
 }
 
 constexpr size_t kScratchBytes =
-    kScratchPartials * sizeof(double) + kScratchGemmFloats * sizeof(float) + kScratchSlots * sizeof(uint64_t);
+    kScratchPartials * sizeof(double) + kScratchGemmFloats * sizeof(float) + kScratchSlots * sizeof(uint64_t) +
+    kScratchOwnFloats * sizeof(float);
 
 int ensure_scratch(int dev) {
     std::lock_guard<std::mutex> lock(g_mutex);
@@ -98,7 +99,7 @@ bool recently_written(const void *p, uint64_t bytes) {
     return false;
 }
 
-int after_launch(const char *name, dim3 grid, dim3 block) {
+int after_launch(const char *name, dim3 grid, dim3 block, hipStream_t stream) {
     g_launches.fetch_add(1, std::memory_order_relaxed);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -107,7 +108,7 @@ int after_launch(const char *name, dim3 grid, dim3 block) {
         return (int)e;
     }
     if (sync_after_launch()) {
-        e = hipStreamSynchronize(current_stream());
+        e = hipStreamSynchronize(stream);
         if (e != hipSuccess) {
             set_error_context("HIP: %s <<<(%u,%u),(%u,%u)>>> faulted: %s", name, grid.x, grid.y,
                               block.x, block.y, hipGetErrorString(e));
@@ -136,6 +137,12 @@ int device_scratch(Scratch *out) {
     out->gemm_floats = kScratchGemmFloats;
     out->slots = reinterpret_cast<uint64_t *>(out->gemm + kScratchGemmFloats);
     return 0;
+}
+
+float *null_stream_scratch() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices || g_devices[dev].scratch == nullptr) return nullptr;
+    return reinterpret_cast<float *>(static_cast<char *>(g_devices[dev].scratch) + kScratchBytes) - kScratchOwnFloats;
 }
 
 }  // namespace dkz

@@ -38,16 +38,21 @@
  *     src/layers/pooling.zig: elementwise and broadcast ops bit-exact, the
  *     per-channel and per-row reductions and softmax within 1e-5 relative,
  *     maxpool indices bit-exact.
- *   - The library owns one scratch buffer per device (130.5 MiB), allocated
+ *   - The library owns one scratch buffer per device (194.5 MiB), allocated
  *     and zeroed by dkz_init: the f64 partial sums of the split per-channel
- *     reductions (2 MiB), the partial tiles of a split-K gemm or convolution
- *     weight gradient (128 MiB) and 64-bit slots (512 KiB: one 256-byte
- *     line per channel's meeting slot or arrival counter, and one 128-byte
- *     posting line per workgroup of a one-launch batch-norm pass), through
- *     which a reduction's workgroups hand each other their partial sums.
- *     Ops never allocate, and leave the slots they use at zero. Reductions or
- *     gemms issued concurrently on two streams of one device share that
- *     buffer and race; issue them on one stream (dkz_set_stream).
+ *     reductions (2 MiB), the partial tiles of a gemm or convolution weight
+ *     gradient and a data gradient's flipped weights and partial tiles (128
+ *     MiB), 64-bit slots (512 KiB: one 256-byte line per channel's meeting
+ *     slot or arrival counter, and one 128-byte posting line per workgroup of
+ *     a one-launch batch-norm pass), through which a reduction's workgroups
+ *     hand each other their partial sums, and the partial tiles of convolution
+ *     forwards and 1x1 data gradients on the null stream (64 MiB).
+ *     Ops never allocate, and leave the slots they use at zero. Reductions,
+ *     gemms, weight gradients and data gradients issued concurrently on two
+ *     streams of one device share that buffer and race; issue them on one
+ *     stream (dkz_set_stream). Forwards and 1x1 data gradients do not: they
+ *     may overlap on any streams, host threads and captured graphs, and are
+ *     fastest on the null stream, where a product's K can be split.
  *   - dkz_batchnorm_forward and dkz_batchnorm_backward may run as one launch
  *     whose workgroups meet per channel. A wait there is bounded (about a
  *     second); if it runs out (the GPU did not hold all of the launch's
@@ -148,10 +153,10 @@ const char *dkz_last_error_context(void);
 /* No counterpart in the reference, which always uses the null stream: choose
  * the hipStream_t (passed as void*) that later ops and copies are issued on.
  * NULL selects the null stream again. The choice is process-wide. Split
- * reductions and gemms use the device's one scratch (partials and
- * per-channel counters), so two streams running them at the same time on
- * one device race: switch streams only between such ops, not to overlap
- * them. */
+ * reductions, gemms and the convolution gradients use the device's one
+ * scratch (partials and per-channel counters; not the 1x1 data gradient), so
+ * two streams running them at the same time on one device race: switch
+ * streams only between such ops, not to overlap them. */
 int dkz_set_stream(void *stream);
 void *dkz_get_stream(void);
 
@@ -357,6 +362,7 @@ int dkz_gemm(int ta, int tb, int m, int n, int k, float alpha, const float *a, i
  * and for ksize == 1 it multiplies by the input itself read as a k x n
  * matrix, as the layer does. The im2col operand is gathered inside the
  * product: no workspace. channels and filters must be multiples of groups.
+ * Calls may overlap on any streams, host threads and captured graphs.
  * Results agree with the per-image calls within fp32 summation error. */
 int dkz_convolution_forward(int batch, int groups, int channels, int height, int width, int filters, int ksize,
                             int stride, int pad, const float *weights, const float *input, float *output);
@@ -383,8 +389,8 @@ int dkz_convolution_weight_gradient(int batch, int groups, int channels, int hei
  *                 a k x n matrix (the layer's beta-0 gemm straight into it);
  *     otherwise:  input_delta(i, j) += col2im(weights(j)^T x delta(i, j)).
  * Results agree with the per-image calls within fp32 summation error. Uses
- * the library's scratch (32 Mi floats) for the flipped weights; no
- * workspace. */
+ * the library's scratch (32 Mi floats) for the flipped weights, but for
+ * ksize == 1, whose calls may overlap as forwards may; no workspace. */
 int dkz_convolution_data_gradient(int batch, int groups, int channels, int height, int width, int filters,
                                   int ksize, int stride, int pad, const float *weights, const float *delta,
                                   float *input_delta);
