@@ -172,7 +172,8 @@ int launch_split(const char *name, SplitArgs g, uint32_t z) {
         g.stream_len = t.stream;
         g.stream_slabs = streamed * slabs;
         g.div_tile_slabs = make_fastdiv(slabs);
-        total = t.full_tiles + div_up(g.stream_slabs, t.stream);
+        g.runs = div_up(g.stream_slabs, t.stream);
+        total = t.full_tiles + g.runs;
     }
     DKZ_REQUIRE(total <= 0x7fffffffull);
     const hipStream_t stream = current_stream();
@@ -318,7 +319,6 @@ int dkz_gemm(int ta, int tb, int m, int n, int k, float alpha, const float *a, i
     g.ldc = (uint32_t)ldc;
     g.alpha = alpha;
     g.beta = beta;
-    g.zgroups = 1;
 
     Scratch sc{};
     if (k >= 8 * kBK) DKZ_TRY(device_scratch(&sc));
@@ -363,7 +363,6 @@ int dkz_convolution_forward(int batch, int groups, int channels, int height, int
     g.ldc = (uint32_t)n;
     g.alpha = 1.0f;
     g.beta = 1.0f;
-    g.zgroups = (uint32_t)groups;
     g.a_z = m * k;
     g.b_z = in_group;
     g.c_z = m * n;
@@ -415,7 +414,6 @@ int dkz_convolution_data_gradient(int batch, int groups, int channels, int heigh
     g.b = delta;
     g.m = (uint32_t)cg;
     g.alpha = 1.0f;
-    g.zgroups = (uint32_t)groups;
     g.b_z = m * npos;
     g.c_z = in_group;
     const uint64_t b_img = (uint64_t)groups * m * npos, c_img = (uint64_t)groups * in_group;
@@ -587,7 +585,6 @@ int dkz_convolution_weight_gradient(int batch, int groups, int channels, int hei
     g.alpha = 1.0f;
     g.beta = 1.0f;
     g.partial = sc.gemm;
-    g.zgroups = 1;
     g.krow = (uint32_t)npos;
     g.a_img = (uint64_t)groups * m * npos;
     g.b_img = (uint64_t)groups * in_group;

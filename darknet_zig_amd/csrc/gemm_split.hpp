@@ -99,12 +99,10 @@ struct SplitArgs {
     uint32_t tiles_m, tiles_n, splits, k_chunk;
     // stream_len != 0 (splits 1, one grid row): tiles from full_tiles on are
     // streamed, stream_len slabs of the line (tile, slab) a workgroup.
-    uint32_t full_tiles, stream_len, stream_slabs;  // stream_slabs: the whole line's
+    uint32_t full_tiles, stream_len, stream_slabs, runs;  // stream_slabs: the whole line's; runs: its workgroups
     FastDiv div_tile_slabs;
     uint32_t tile_bm, tile_bn_log2;
-    // Batched launches (z = blockIdx.y): A at a + (z % zgroups) * a_z, B at
-    // b + z * b_z, C at c + z * c_z.
-    uint32_t zgroups;
+    // Groups (z = blockIdx.y): A at a + z * a_z, B at b + z * b_z, C at c + z * c_z.
     uint64_t a_z, b_z, c_z;
     // Columns over (image, position): npos positions per image (0: one matrix),
     // element strides from one image to the next of B and C.
@@ -602,12 +600,13 @@ constexpr int min_waves() { return BM * BN >= 128 * 128 ? 2 : BM * BN >= 128 * 6
 // registers; a 128x128 tile's would take 128), each a part of the g.tile_bm x
 // g.tile_bn tile whose pieces it adds up, or the 32x128 ones.
 template <int BM, int BN, Operand AK, Operand BK, bool ORDERED = false>
-__global__ __launch_bounds__(kBlock, (min_waves<BM, BN>() - (ORDERED ? 1 : 0))) void gemm_split_kernel(SplitArgs g) {
+__global__ __launch_bounds__(kBlock, (min_waves<BM, BN>() - (ORDERED ? 2 : 0))) void gemm_split_kernel(SplitArgs g) {
     constexpr int kRowsOfWaves = BM == 32 ? 1 : 2;  // 32-row tiles: four waves side by side
     constexpr int WM = BM / kRowsOfWaves, WN = BN * kRowsOfWaves / 4, TM = WM / 32, TN = WN / 32;
     constexpr int RA = BM == 32 ? 64 : BM;  // rows of A staged (of a 32-row tile, the last row again)
     constexpr int kA = slab_words<RA>(), kB = slab_words<BN>();
     __shared__ __align__(16) uint32_t lds[2 * (kA + kB)];
+    __shared__ uint32_t votes[kBlock / kWave];
     static_assert((RA + BN) * kF32Pitch <= 2 * (kA + kB), "the fp32 pass uses the same LDS");
 
     constexpr bool kGa = BK == kGather || BK == kGatherWide;
@@ -638,7 +637,7 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>() - (ORDERED ? 1 : 0))) 
         k_chunk = lda = k_all;
         a_z = (uint64_t)g.m * k_all;
     }
-    const float *ga = a_base + (size_t)(z % g.zgroups) * a_z;
+    const float *ga = a_base + (size_t)z * a_z;
     const float *gb = g.b + (size_t)z * g.b_z;
     float *gc = g.c + (size_t)z * g.c_z;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -667,7 +666,7 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>() - (ORDERED ? 1 : 0))) 
         line = g.stream_len != 0 ? block * slabs : 0;
         line_end = line + slabs;
     } else if (streams) {
-        block = xcd_order(block - g.full_tiles, gridDim.x - g.full_tiles);
+        block = xcd_order(block - g.full_tiles, g.runs);
         line = block * g.stream_len;
         line_end = min(line + g.stream_len, g.stream_slabs);
     }
@@ -792,11 +791,13 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>() - (ORDERED ? 1 : 0))) 
             DKZ_SPLIT_SCHED();
             __syncthreads();
         };
+        // One slab alone loads no others (where registers are left for the branches).
+        constexpr bool kLean = kQuads && TM * TN == 1;
         load(0, slab_k(0));
         if (tail && whole == 1) load_tail(1, kbeg + kBK);  // a first layer's 27 k: both slabs at once
-        else load(1, slab_k(1));
+        else if (!kLean || whole > 1) load(1, slab_k(1));
         store(0);
-        load(0, slab_k(2));
+        if (!kLean || whole > 1) load(0, slab_k(2));
         __syncthreads();
         uint32_t s = 0;
 #pragma unroll 1
@@ -832,7 +833,11 @@ __global__ __launch_bounds__(kBlock, (min_waves<BM, BN>() - (ORDERED ? 1 : 0))) 
 #pragma unroll
             for (int r = 0; r < 16; ++r) redo |= !(fabsf(big[ti][tj][r]) < __builtin_inff());
         }
-    if (__syncthreads_or(redo)) {
+    // One barrier (__syncthreads_or takes three, and a load of the workgroup's size).
+    const bool any = __builtin_amdgcn_ballot_w64(redo) != 0;
+    if (lane == 0) votes[wave] = any;
+    __syncthreads();
+    if ((votes[0] | votes[1] | votes[2] | votes[3]) != 0) {
         float *as = reinterpret_cast<float *>(lds), *bs = as + RA * kF32Pitch;
 #pragma unroll
         for (int ti = 0; ti < TM; ++ti)
