@@ -4,6 +4,8 @@
 //   * chk_fastdiv: the launch-constant division, run on the host;
 //   * chk_xcd_run_block: the workgroup renumbering that keeps runs of
 //     logical blocks on one XCD, run on the host;
+//   * chk_pick_tiling: which tiles and K ranges a matrix product runs in
+//     (darknet_zig_amd/csrc/gemm_tiling.hpp), on the host;
 //   * chk_exp2f_tab: the expf table entries, for the high-precision check;
 //   * chk_expf_host_mismatches: expf_libm compiled for the host, compared
 //     with the C library's expf over a range of float bit patterns;
@@ -25,6 +27,7 @@
 #include <vector>
 
 #include "dkz_device.hpp"
+#include "gemm_tiling.hpp"
 
 namespace {
 
@@ -143,6 +146,12 @@ extern "C" {
 uint32_t chk_fastdiv(uint32_t n, uint32_t d) { return dkz::fdiv(n, dkz::make_fastdiv(d)); }
 
 uint32_t chk_xcd_run_block(uint32_t b, uint32_t grid, uint32_t r) { return dkz::xcd_run_block(b, grid, r); }
+
+void chk_pick_tiling(uint64_t m, uint64_t n, uint64_t k, uint64_t z, uint64_t partial_floats, int wide, uint32_t *out) {
+    const dkz::Tiling t = dkz::pick_tiling(m, n, k, z, partial_floats, wide != 0);
+    const uint32_t v[6] = {t.bm, t.bn, t.splits, t.k_chunk, t.full_tiles, t.stream};
+    memcpy(out, v, sizeof v);
+}
 
 uint64_t chk_exp2f_tab(uint32_t i) { return dkz::exp2f_tab(i); }
 

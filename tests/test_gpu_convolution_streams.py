@@ -15,23 +15,38 @@ import pytest
 from darknet_zig_amd import _lib, gpu
 from oracle import ref
 from tests.helpers import down, rng, up
+from tests.tilings import OWN, tiling
 from tests.test_gpu_streams_graphs import Hip, quiet  # noqa: F401  (quiet: a fixture)
 
 pytestmark = pytest.mark.gpu
 
-FORWARDS = [
-    # batch, groups, channels, height, width, filters, ksize, stride, pad
-    (1, 1, 64, 52, 52, 128, 3, 1, 1),    # 64x64 tiles, four ranges of K
-    (1, 1, 512, 13, 13, 96, 3, 1, 1),    # the last range shorter
-    (1, 1, 512, 7, 7, 10, 1, 1, 0),      # ksize 1, 32 rows
-    (39, 1, 263, 13, 13, 153, 3, 1, 1),  # streamed, partial tiles
-    (40, 1, 128, 40, 40, 130, 3, 1, 1),  # whole rounds of tiles, then streamed ones
-    (1, 1, 3, 40, 40, 64, 33, 1, 2),     # 64-bit gathers, ranges of K
-    (4, 1, 64, 26, 26, 32, 3, 1, 1),
-    (2, 2, 64, 9, 9, 72, 3, 1, 1),       # groups: K whole
-    (2, 1, 3, 33, 31, 20, 3, 1, 1),      # 27 k
-]
-DATA_GRADIENTS = [(1, 1, 96, 13, 13, 1024, 1, 1, 0), (33, 1, 250, 13, 13, 1000, 1, 1, 0), (2, 1, 40, 7, 7, 300, 1, 1, 0)]
+FORWARDS = {
+    # batch, groups, channels, height, width, filters, ksize, stride, pad: the product's tiles
+    (1, 1, 64, 52, 52, 128, 3, 1, 1): "64x64 ranges",
+    (1, 1, 512, 13, 13, 96, 3, 1, 1): "64x64 ranges",
+    (1, 1, 512, 7, 7, 10, 1, 1, 0): "64x64 ranges",
+    (7, 1, 195, 32, 19, 17, 1, 1, 0): "32x128 ranges",
+    (10, 1, 50, 31, 36, 34, 3, 1, 1): "64x128 ranges",
+    (8, 1, 80, 29, 26, 97, 3, 1, 1): "128x64 ranges",
+    (39, 1, 88, 6, 48, 68, 3, 1, 1): "128x128 ranges",
+    (39, 1, 263, 13, 13, 153, 3, 1, 1): "32x128 streamed",
+    (53, 1, 38, 58, 44, 18, 3, 1, 1): "32x128 rounds, then streamed",
+    (15, 1, 126, 41, 18, 165, 3, 1, 1): "64x64 streamed",
+    (13, 1, 34, 54, 47, 99, 3, 1, 1): "64x64 rounds, then streamed",
+    (18, 1, 121, 51, 36, 37, 3, 1, 1): "64x128 streamed",
+    (44, 1, 35, 46, 50, 45, 3, 1, 1): "64x128 rounds, then streamed",
+    (37, 1, 151, 11, 41, 118, 3, 1, 1): "128x128 streamed",
+    (45, 1, 172, 49, 30, 99, 1, 1, 0): "128x128 rounds, then streamed",
+    (1, 1, 3, 40, 40, 64, 33, 1, 2): "64x64 ranges",  # 64-bit gathers
+    (4, 1, 64, 26, 26, 32, 3, 1, 1): "32x128 ranges",
+    (2, 2, 64, 9, 9, 72, 3, 1, 1): "64x64 whole",     # groups
+    (2, 1, 3, 33, 31, 20, 3, 1, 1): "64x64 whole",    # 27 k
+}
+DATA_GRADIENTS = {
+    (1, 1, 96, 13, 13, 1024, 1, 1, 0): "64x64 ranges",
+    (45, 1, 99, 49, 30, 172, 1, 1, 0): "128x128 rounds, then streamed",
+    (2, 1, 40, 7, 7, 300, 1, 1, 0): "64x64 ranges",
+}
 
 
 def _buffers(case, seed):
@@ -56,6 +71,13 @@ def _plans():
     return [(c, _forward) for c in FORWARDS] + [(c, _data_gradient) for c in DATA_GRADIENTS]
 
 
+def _kind(case, op):
+    batch, groups, cin, H, W, F, ks, s, p = case
+    n = batch * ref.conv_out_dim(H, ks, s, p) * ref.conv_out_dim(W, ks, s, p)
+    m, k = (F, cin * ks * ks) if op is _forward else (cin, F)
+    return tiling(m // groups, n, k // groups, groups, OWN, wide=ks > 32).kind
+
+
 def _setup(case, op, seed=1):
     x, w, d = _buffers(case, seed)
     src, other = (x, d) if op is _forward else (d, x)
@@ -71,6 +93,7 @@ def _stream(hip):
 
 @pytest.mark.parametrize("case,op", _plans(), ids=lambda v: v.__name__ if callable(v) else str(v))
 def test_same_on_every_stream_and_in_a_graph(quiet, case, op):  # noqa: F811
+    assert _kind(case, op) == (FORWARDS if op is _forward else DATA_GRADIENTS)[case]
     hip = Hip()
     src, w, other, out = _setup(case, op)
     like = np.empty(out.len, np.float32)
@@ -111,7 +134,8 @@ def test_overlapping_streams(quiet):  # noqa: F811
     """Three streams (the null one among them), each with its own layer and
     buffers, fed in turn without waiting: twenty accumulated passes each."""
     hip = Hip()
-    plans = [(FORWARDS[0], _forward), (FORWARDS[3], _forward), (DATA_GRADIENTS[1], _data_gradient)]
+    plans = [((1, 1, 64, 52, 52, 128, 3, 1, 1), _forward), ((39, 1, 263, 13, 13, 153, 3, 1, 1), _forward),
+             ((45, 1, 99, 49, 30, 172, 1, 1, 0), _data_gradient)]
     state = [_setup(c, op, 3 + i) for i, (c, op) in enumerate(plans)]
     want = []
     for (case, op), (src, w, _, out) in zip(plans, state):
@@ -144,7 +168,7 @@ def test_two_threads_on_the_null_stream(quiet):  # noqa: F811
     """Two host threads, each with its own layer: a product and its reduction
     stay together."""
     import threading
-    plans = [(FORWARDS[0], _forward), (FORWARDS[1], _forward)]
+    plans = [((1, 1, 64, 52, 52, 128, 3, 1, 1), _forward), ((1, 1, 512, 13, 13, 96, 3, 1, 1), _forward)]
     state = [_setup(c, op, 7 + i) for i, (c, op) in enumerate(plans)]
     errors = []
 

@@ -17,12 +17,24 @@ import pytest
 from darknet_zig_amd import gpu
 from tests.helpers import rng
 from tests.test_gpu_gemm import VARIANTS, bound, layout, run_gpu
+from tests.tilings import tiling
 
 pytestmark = pytest.mark.gpu
 
-# 64x64 tiles in one K range and in several, 128x128 tiles with 1, 16 and 17 k
-# (no whole slab, one, one and a tail), and in two K ranges; odd rows and columns.
-SHAPES = [(3, 5, 7), (65, 130, 300), (2049, 4100, 1), (2049, 4100, 16), (2050, 4099, 17), (2047, 2050, 1030)]
+# Tiles with 1, 16 and 17 k (no whole slab, one, one and a tail), K whole and in
+# ranges; odd rows and columns.
+SHAPES = {
+    (3, 5, 7): "64x64 whole",
+    (65, 130, 300): "64x64 ranges",
+    (2049, 4100, 1): "128x64 whole",
+    (2049, 4100, 16): "128x64 whole",
+    (2050, 4099, 17): "128x64 whole",
+    (1385, 4458, 1): "128x128 whole",
+    (1385, 4458, 16): "128x128 whole",
+    (1385, 4458, 17): "128x128 whole",
+    (2047, 2047, 2300): "128x128 ranges",
+    (2047, 2050, 1030): "128x128 streamed",
+}
 
 
 def product(A, B, ta=False, tb=False):
@@ -51,6 +63,7 @@ def check(A, B, ta=False, tb=False):
 @pytest.mark.parametrize("m,n,k", SHAPES)
 @pytest.mark.parametrize("ta,tb", VARIANTS)
 def test_shapes(dev, ta, tb, m, n, k):
+    assert tiling(m, n, k).kind == SHAPES[m, n, k]
     r = rng(m + n + k)
     check(r.normal(size=(m, k)).astype(np.float32), r.normal(size=(k, n)).astype(np.float32), ta, tb)
 
@@ -59,6 +72,7 @@ def test_shapes(dev, ta, tb, m, n, k):
 def test_k_in_ranges(dev, m, n, k):
     """16, 79 and 448 partials, one and sixteen lanes an output, in float4s and
     floats."""
+    assert tiling(m, n, k).splits in (16, 79, 447, 448)
     r = rng(m + n + k)
     check(r.normal(size=(m, k)).astype(np.float32), r.normal(size=(k, n)).astype(np.float32))
 

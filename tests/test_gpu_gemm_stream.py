@@ -15,18 +15,20 @@ from tests import test_gpu_convolution as base
 from tests.helpers import rng
 from tests.test_gpu_gemm import VARIANTS
 from tests.test_gpu_gemm_split import check
+from tests.tilings import OWN, SHARED, tiling
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (1652, 2625, 823),  # 273 tiles of 128x128, 28 slabs a run of tiles of 52
-    (2403, 3416, 164),  # 512 tiles, then one streamed in runs of four slabs
-    (802, 4997, 305),   # 1024 tiles of 64x64 first
-    (1281, 3146, 313),  # 1024 tiles of 32x128 first
+@pytest.mark.parametrize("m,n,k,kind", [
+    (1652, 2625, 823, "128x128 streamed"),               # 273 tiles, 28 slabs a run of tiles of 52
+    (2403, 3416, 164, "128x128 rounds, then streamed"),  # 512 tiles, then one streamed in runs of four slabs
+    (802, 4997, 305, "64x64 rounds, then streamed"),     # 1024 tiles first
+    (1281, 3146, 313, "32x128 rounds, then streamed"),   # 1024 tiles first
 ])
 @pytest.mark.parametrize("ta,tb", VARIANTS)
-def test_gemm(dev, ta, tb, m, n, k):
+def test_gemm(dev, ta, tb, m, n, k, kind):
+    assert tiling(m, n, k).kind == kind
     r = rng(m + n + k)
     check(r.normal(size=(m, k)).astype(np.float32), r.normal(size=(k, n)).astype(np.float32), ta, tb)
 
@@ -42,14 +44,20 @@ def test_gemm_with_an_infinity(dev):
 
 @pytest.mark.parametrize("case", [(39, 1, 263, 13, 13, 153, 3, 1, 1), (37, 1, 156, 14, 14, 158, 3, 1, 1)], ids=str)
 def test_forward(dev, case):
+    b, _, c, h, w, f, ks, _, _ = case
+    assert "streamed" in tiling(f, b * h * w, c * ks * ks, floats=OWN).kind
     base.test_convolution_forward(dev, case)
 
 
 @pytest.mark.parametrize("case", [(21, 1, 254, 13, 13, 366, 3, 1, 1), (39, 1, 300, 14, 14, 133, 3, 1, 1)], ids=str)
 def test_weight_gradient(dev, case):
+    b, _, c, h, w, f, ks, _, _ = case
+    assert "streamed" in tiling(f, c * ks * ks, b * ((h * w + 3) // 4 * 4)).kind
     base.test_convolution_weight_gradient(dev, case)
 
 
 @pytest.mark.parametrize("case", [(32, 1, 134, 13, 13, 360, 3, 1, 1), (37, 1, 133, 14, 14, 182, 3, 1, 1)], ids=str)
 def test_data_gradient(dev, case):
+    b, _, c, h, w, f, ks, _, _ = case  # the partials lie behind the flipped weights
+    assert "streamed" in tiling(c, b * h * w, f * ks * ks, floats=SHARED - (f * c * ks * ks + 63) // 64 * 64).kind
     base.test_convolution_data_gradient(dev, case)
