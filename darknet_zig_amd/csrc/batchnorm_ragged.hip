@@ -385,7 +385,12 @@ bool forward(const FwdArgs &a, int *rc) {
     FwdFin fin{nullptr, a.mean, a.variance, a.rolling_mean, a.rolling_variance, (double)L, 1.0f / (float)L,
                1.0f / (float)(L - 1u)};
     // The channel in one workgroup's registers where it fits (the smallest
-    // workgroup that holds it), except for the largest tensors.
+    // workgroup that holds it), except for the largest tensors. With few
+    // channels that leaves CUs idle, but is well ahead of the per-op sequence at
+    // every count: [32,F,75,75] forward 35.5 / 50.5 / 76.9 / 127 / 246 us in the
+    // sequence and 9.8 / 15.5 / 26.9 / 41.8 / 84.1 so, backward 31.5 / 49.2 / 69.8
+    // / 121 / 201 and 12.8 / 22.1 / 40.1 / 67.2 / 123, for F = 1, 16, 32, 64, 128;
+    // [1,F,207,207] forward 39 and 16 to 19 us for F up to 64.
     const RedGeom whole = make_red_geom(sh.F, sh.S, L, 1, false);
     if (chan_fits(sh, 64 * 1024) && (sh.n <= kMaxOneLaunch || !apply)) {
         if (L <= 4 * 256) *rc = fwd_chan_launch<A, 256, 4>(a, whole, fin);

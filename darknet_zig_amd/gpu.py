@@ -88,7 +88,7 @@ def deviceMemoryMib() -> int:  # gpu.zig:153-155
 
 
 def gemmPolicy() -> str:
-    """gpu.zig:104-108: the GEMM a run uses (the library's fp32 matrix-core
+    """gpu.zig:104-108: the GEMM a run uses (the library's matrix-core
     kernel), "cpu" when no device is active."""
     return "dkz-mfma" if active() else "cpu"
 

@@ -87,7 +87,7 @@ inline int device_index = -1;
 inline bool active() { return enabled && device_index >= 0; }
 
 // gpu.zig:104-113: the GEMM a run uses, for a benchmark record -- the
-// library's fp32 matrix-core kernel ("cpu" when no device is active) -- and
+// library's matrix-core kernel ("cpu" when no device is active) -- and
 // the tile threshold the reference's blocked kernel was gated on, which the
 // library does not have (0).
 inline const char *gemmPolicy() { return active() ? "dkz-mfma" : "cpu"; }

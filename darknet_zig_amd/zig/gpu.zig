@@ -51,7 +51,7 @@ inline fn ci(x: usize) c_int {
 }
 
 /// gpu.zig:104-108: which GEMM a GPU run uses, for the benchmark to record.
-/// The library has one, on the fp32 matrix cores; "cpu" when no device is
+/// The library has one, on the matrix cores; "cpu" when no device is
 /// active, as in the reference.
 pub fn gemmPolicy() []const u8 {
     if (!active()) return "cpu";

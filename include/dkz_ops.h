@@ -342,9 +342,11 @@ int dkz_col2im(const float *col, int channels, int height, int width, int ksize,
 /* gpu.zig:671-719 gemm(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc):
  * C = alpha*op(A)*op(B) + beta*C, all row-major; op(A) is m x k (A is k x m
  * with leading dimension lda when ta != 0), op(B) is k x n. beta == 0 clears
- * C first (NaN included), beta != 1 scales it (gemm.zig:121-131). fp32
- * products and sums on the matrix cores: results agree with the CPU twin
- * within fp32 summation error. m == 0 or n == 0 does nothing (gpu.zig:686);
+ * C first (NaN included), beta != 1 scales it (gemm.zig:121-131). Products
+ * are made of six bf16 ones on the matrix cores and are within 2^-24 of the
+ * exact ones, sums are fp32 (f64 between ranges of k): results agree with the
+ * CPU twin within fp32 summation error, and infinities, NaNs and tiny values
+ * give what fp32 products give. m == 0 or n == 0 does nothing (gpu.zig:686);
  * a leading dimension below the row length is hipErrorInvalidValue.
  * gemm.zig:47-278 */
 int dkz_gemm(int ta, int tb, int m, int n, int k, float alpha, const float *a, int lda, const float *b,
@@ -415,8 +417,9 @@ int dkz_adam_update(float *w, float *d, float *m, float *v, float b1, float b2, 
  * per-op entry points stay. Results equal the sequence's: every element
  * expression is the same op's, in the same order, given the same per-channel
  * values; the per-channel sums are the channel reductions' (within 1e-5 of
- * the CPU twin, or closer to the exact value). Shapes with spatial % 4 != 0,
- * empty tensors or tensors not 16-byte aligned run the per-op sequence. */
+ * the CPU twin, or closer to the exact value). Empty tensors, large ones with
+ * rows of under four floats and large ones not 16-byte aligned run the per-op
+ * sequence. */
 
 /* Forward of a batch-normalised layer and its activation: the sequence of
  * layers/batchnorm.zig:129-153 (forwardGpu) followed by
