@@ -5,7 +5,8 @@
 // bits each, rounded to nearest, so 24 bits in all): exact for |x| >= 2^-109.
 // A product of two such sums keeps six of its nine terms,
 //     hh | hm + mh + mm + hl + lh,
-// the rest (ml, lm, ll) being up to 2^-24 of it, 2^-27.5 rms. v_mfma_f32_32x32x16_bf16 forms the
+// the rest (ml, lm, ll) being up to 2^-24 of it, 2^-27.5 rms.
+// v_mfma_f32_32x32x16_bf16 forms the
 // products exactly and adds them in fp32, rounding twice per 16 k. hh has an
 // accumulator of its own and the five small terms another, so the large one is
 // rounded once per 8 k (the fp32 matrix instruction rounds it at every k): over

@@ -1,9 +1,9 @@
 """dkz_gemm's split of fp32 operands into three bf16 values each (h + m + l).
 
 Six of the nine products are kept; what the split cannot hold -- infinities,
-NaNs, values that round to a bf16 infinity, rows of values so small that l (or
-m) falls below bf16's smallest denormal -- goes through the fp32 matrix
-instruction, tile by tile. Tolerance for finite results: Higham's bound for any
+NaNs, values that round to a bf16 infinity, values so small that l (or m, or h)
+falls below bf16's smallest denormal -- goes through the fp32 matrix
+instruction, tile by tile, and so do products with one k. Tolerance for finite results: Higham's bound for any
 fp32 summation order, gamma_(k+3) * sum |a||b| (as in test_gpu_gemm), plus
 k * 2^-149 for products below fp32's range. Infinities and NaNs must be where
 IEEE arithmetic on the same operands puts them.
